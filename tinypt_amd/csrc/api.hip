@@ -676,7 +676,7 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
         const int j = nsets == 2 ? (int)(pass & 1) : 0;
         PathSet* S = &c->set[j];
         uint32_t kk = std::min(k, spp - s0);
-        PassArgs A{np * kk, np, p0, s0, nullptr, nullptr, pix_map};
+        PassArgs A{np * kk, np, kk, p0, s0, nullptr, nullptr, pix_map};
         rc = wf_bounces(S, W[j], A, *tt[j], &launches);
         if (rc) return rc;
         AccumArgs B{np, p0, kk, acc, acc_w, acc_sq};
@@ -720,7 +720,7 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
       for (uint32_t c0 = 0; c0 < n_active; c0 += chunk, j ^= 1) {
         PathSet* S = &c->set[j];
         const uint32_t nc = std::min(chunk, n_active - c0);
-        PassArgs A{nc * kk, nc, 0, 0, act_in + c0, c->nsamp.as<uint32_t>(), pix_map};
+        PassArgs A{nc * kk, nc, kk, 0, 0, act_in + c0, c->nsamp.as<uint32_t>(), pix_map};
         rc = wf_bounces(S, W[j], A, *tt[j], &launches);
         if (rc) return rc;
         AdaptiveArgs B{nc, kk, min_spp, spp, cfg->adaptive_threshold, act_in + c0, act_out, n_out,

@@ -1,8 +1,8 @@
 // k_wavefront.hip -- FP32 wavefront path tracer (radiance(), integrator.rs:53-135, split into
 // kernels over SoA path queues).
 //
-// One pass renders `k` samples of a set of pixels: P = pixels * k paths, slot i -> pixel
-// (i mod pixels), sample (s0 + i / pixels), so neighbouring slots are neighbouring pixels.
+// One pass renders `k` samples of a set of pixels: P = pixels * k paths, slot i -> pixel and
+// sample by path_pixel (wavefront.h), so that neighbouring slots are samples of the same pixels.
 // Per bounce:  extend (closest hit) -> shade (miss / RR / emission / NEE sampling / BSDF
 // sampling; survivors compacted into the next queue) -> light self-occlusion -> shadow (any hit
 // for the <= 2 NEE rays of each path, added to that path's radiance by the thread that owns the
@@ -68,13 +68,13 @@ __device__ __forceinline__ uint32_t gtid() { return blockIdx.x * blockDim.x + th
 // kernels call it for their own paths, so no path state is written for bounce 0.
 __device__ __forceinline__ void gen_path(const WfParams& W, const PassArgs& A, uint32_t i, RngF32* rng, f3* o, f3* d) {
   uint32_t pix, s;
+  path_pixel(i, A.n_pixels, A.k, &pix, &s);
   if (A.active) {
-    const uint32_t j = i % A.n_pixels;
-    pix = (uint32_t)A.active[j];
-    s = A.nsamp[pix] + i / A.n_pixels;
+    pix = (uint32_t)A.active[pix];
+    s += A.nsamp[pix];
   } else {
-    pix = A.pixel0 + i % A.n_pixels;
-    s = A.s0 + i / A.n_pixels;
+    pix += A.pixel0;
+    s += A.s0;
   }
   if (A.pix_map) pix = (uint32_t)A.pix_map[pix];
   const uint32_t x = pix % (uint32_t)W.width, y = pix / (uint32_t)W.width;
@@ -482,12 +482,14 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_
               (unsigned long long)tot);
 }
 
-// Non-adaptive: pixel p accumulates the k paths of this pass (slots p + j * pixels).
+// Non-adaptive: pixel p accumulates the k paths of this pass, in sample order.
 __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate(WfParams W, AccumArgs A) {
   for (uint32_t p = gtid(); p < A.n_pixels; p += gridDim.x * blockDim.x) {
     double r = 0, g = 0, b = 0, r2 = 0, g2 = 0, b2 = 0;
+    uint32_t first, step;
+    path_index(p, A.n_pixels, A.k, &first, &step);
     for (uint32_t j = 0; j < A.k; j++) {
-      float4 l = W.ps.L[p + j * A.n_pixels];
+      float4 l = W.ps.L[first + j * step];
       double x = l.x, y = l.y, z = l.z;
       r += x; g += y; b += z;
       r2 += x * x; g2 += y * y; b2 += z * z;
@@ -518,8 +520,10 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate_adaptive(WfParams W
       double mean = A.welford[2 * pix], m2 = A.welford[2 * pix + 1];
       double r = 0, g = 0, b = 0, r2 = 0, g2 = 0, b2 = 0;
       bool stop = false;
+      uint32_t first, step;
+      path_index(j, A.n_active, A.k, &first, &step);
       for (uint32_t k = 0; k < A.k && !stop; k++) {
-        float4 l = W.ps.L[j + k * A.n_active];
+        float4 l = W.ps.L[first + k * step];
         double x = l.x, y = l.y, z = l.z;
         r += x; g += y; b += z;
         r2 += x * x; g2 += y * y; b2 += z * z;

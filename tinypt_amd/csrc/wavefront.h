@@ -127,11 +127,42 @@ struct WfParams {
   int32_t pad;
 };
 
-// The paths of one pass: path i is pixel (i mod n_pixels) of the pass's pixel set, sample
-// (i / n_pixels) of the samples the pass adds to it.
+// Path order of a pass of n_pixels pixels and k samples: the pixels in groups of TPT_WF_PIX_GROUP
+// (the last one may hold fewer), a group's paths together, sample after sample.  A wave's 64
+// camera rays then start in a few pixels and the rays in flight on the chip cover a small part of
+// the image, so they meet the same nodes, triangles and materials; sample-major order (path i is
+// pixel i mod n_pixels) had the whole image in flight.  Groups of 2 measured best (against
+// sample-major order on MI355X: default scene 256^2 x 64 spp 873 -> 759 us, Cornell 512^2 x 256 spp
+// 28.5 -> 27.85 ms, 1.31M-triangle mesh 1080p x 32 spp 47.5 -> 44.7 ms, 4096 instances adaptive
+// 56.2 -> 53.5 ms; groups of 4 781 us, 27.95, 44.9, 54.2; of 16 787 us, 27.9, 45.6, 55.6; one pixel
+// at a time reads the sums uncoalesced: Cornell 28.1).
+#define TPT_WF_PIX_GROUP 2
+// Path i: pixel `pix` of the pass's pixel set, sample `s` of the samples the pass adds to it.
+__host__ __device__ __forceinline__ void path_pixel(uint32_t i, uint32_t n_pixels, uint32_t k, uint32_t* pix,
+                                                    uint32_t* s) {
+  const uint32_t g = i / (TPT_WF_PIX_GROUP * k), r = i - g * (TPT_WF_PIX_GROUP * k);
+  const uint32_t p0 = g * TPT_WF_PIX_GROUP, left = n_pixels - p0;
+  if (left >= TPT_WF_PIX_GROUP) {
+    *pix = p0 + r % TPT_WF_PIX_GROUP;
+    *s = r / TPT_WF_PIX_GROUP;
+  } else {
+    *pix = p0 + r % left;
+    *s = r / left;
+  }
+}
+// First path of pixel `pix` and the stride between its samples' paths.
+__host__ __device__ __forceinline__ void path_index(uint32_t pix, uint32_t n_pixels, uint32_t k, uint32_t* first,
+                                                    uint32_t* stride) {
+  const uint32_t p0 = pix / TPT_WF_PIX_GROUP * TPT_WF_PIX_GROUP, left = n_pixels - p0;
+  *first = p0 * k + (pix - p0);
+  *stride = left >= TPT_WF_PIX_GROUP ? TPT_WF_PIX_GROUP : left;
+}
+
+// The paths of one pass, in the order above.
 struct PassArgs {
   uint32_t n_paths;   // pixels * k
   uint32_t n_pixels;  // pixels in this pass
+  uint32_t k;         // samples of each pixel
   uint32_t pixel0;    // first pixel (non-adaptive)
   uint32_t s0;        // first sample index (non-adaptive)
   const int32_t* active;  // adaptive: active pixel list (else null)
