@@ -2,10 +2,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/tinypt_gpu.h"
@@ -92,6 +94,9 @@ struct PathSet {
   DevBuf ps_o[2], ps_d[2], ps_beta[2], ps_rng[2], ps_hit, ps_L, sh_o[2], sh_d[2], sh_c[2], sh_l, sh_lv, shl_keep, counters,
       stats, gstack;
   size_t ps_cap = 0;
+  uint64_t* seen = nullptr;  // pinned word in which a bounce's extension reports its path count (PathCount)
+  uint64_t* seen_dev = nullptr;  // its device address
+  uint32_t seen_tag = 0;         // tag of the last report asked for
   EventPool ev_trace;  // timing events of the extension launches (one call at a time)
   hipEvent_t done = nullptr;  // recorded after the set's last accumulation of a render
 };
@@ -201,7 +206,12 @@ int tpt_ctx_create(int device, tpt_ctx** out) {
   HIPC(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   c->set[0].stream = c->stream;
   HIPC(hipStreamCreateWithFlags(&c->set[1].stream, hipStreamNonBlocking));
-  for (PathSet& ps : c->set) HIPC(hipEventCreateWithFlags(&ps.done, hipEventDisableTiming));
+  for (PathSet& ps : c->set) {
+    HIPC(hipEventCreateWithFlags(&ps.done, hipEventDisableTiming));
+    HIPC(hipHostMalloc((void**)&ps.seen, 64, hipHostMallocMapped | hipHostMallocCoherent));
+    *ps.seen = 0;
+    HIPC(hipHostGetDevicePointer((void**)&ps.seen_dev, ps.seen, 0));
+  }
   *out = c.release();
   return TPT_OK;
 }
@@ -212,6 +222,7 @@ int tpt_ctx_destroy(tpt_ctx* ctx) {
   for (PathSet& ps : ctx->set) {
     if (ps.stream) (void)hipStreamSynchronize(ps.stream);
     if (ps.done) (void)hipEventDestroy(ps.done);
+    if (ps.seen) (void)hipHostFree(ps.seen);
   }
   if (ctx->set[1].stream) (void)hipStreamDestroy(ctx->set[1].stream);
   (void)hipStreamDestroy(ctx->stream);
@@ -594,27 +605,121 @@ struct EventTimer {
   }
 };
 
-// Bounce loop of one pass over the A.n_paths paths that A describes; the first bounce's kernels
-// generate the camera rays themselves.
-int wf_bounces(PathSet* c, const WfParams& W, const PassArgs& A, EventTimer& tt, uint64_t* launches) {
-  hipStream_t s = c->stream;
-  const uint32_t P = A.n_paths;
-  if ((size_t)P > c->ps_cap) return fail(TPT_ERR_INTERNAL, "a pass holds more paths than were allocated");
-  if (W.max_bounces == 0) HIPC(wf_launch_clear_radiance(W, P, s));
-  int cur = 0;
-  for (int b = 0; b < W.max_bounces; b++) {
-    const PassArgs* gen = b == 0 ? &A : nullptr;
+// The bounce loop of one pass over the A.n_paths paths that A describes, in steps so that one host
+// thread can drive a pass on each path set: the first bounce's kernels generate the camera rays
+// themselves; every later bounce's path count is reported to the host when the kernels after its
+// predecessor's shading start (PathCount), and once few paths are left one k_tail launch takes them
+// to their ends.
+struct PassRun {
+  PathSet* c = nullptr;
+  const WfParams* W = nullptr;
+  EventTimer* tt = nullptr;
+  PassArgs A{};
+  int b = 0, cur = 0;    // the next bounce to shade (its extension is queued) and its path queue
+  bool running = false;  // bounces are left to queue
+  int known_b = 0;       // the last bounce whose path count is known ...
+  uint32_t known_n = 0;  // ... and that count
+  uint32_t tag0 = 0;     // tag of bounce 0
+  uint32_t polls = 0;    // since the last launch
+
+  int extend(const PassArgs* gen, const PathCount& count, uint64_t* launches) {
     hipEvent_t e0, e1;
-    HIPC(tt.reserve_pair(&e0, &e1));
-    HIPC(wf_launch_extend(W, cur, gen, P, s, e0, e1));
+    HIPC(tt->reserve_pair(&e0, &e1));
+    HIPC(wf_launch_extend(*W, cur, gen, count, known_n, c->stream, e0, e1));
     (*launches)++;
-    HIPC(wf_launch_shade(W, cur, gen, P, s));
-    if (W.lights.n > 0) {
-      HIPC(wf_launch_light_selfocc(W, cur, gen, P, s));
-      HIPC(wf_launch_shadow(W, 1, P, s));
+    return TPT_OK;
+  }
+  // The rest of bounce b, then the next bounce's extension.
+  int shade(const PassArgs* gen, uint64_t* launches) {
+    hipStream_t s = c->stream;
+    const bool last = b + 1 >= W->max_bounces;
+    const PathCount count{last ? nullptr : c->seen_dev, tag0 + (uint32_t)b + 1, cur ^ 1};
+    HIPC(wf_launch_shade(*W, cur, gen, known_n, s));
+    if (W->lights.n > 0) {
+      HIPC(wf_launch_light_selfocc(*W, cur, gen, count, known_n, s));
+      HIPC(wf_launch_shadow(*W, 1, count, known_n, s));
     }
-    if (W.env.kind == TPT_ENV_IMAGE && !W.env.black) HIPC(wf_launch_shadow(W, 0, P, s));
+    if (W->env.kind == TPT_ENV_IMAGE && !W->env.black) HIPC(wf_launch_shadow(*W, 0, count, known_n, s));
     cur ^= 1;
+    b++;
+    running = !last;
+    polls = 0;
+    return running ? extend(nullptr, count, launches) : TPT_OK;
+  }
+  int start(PathSet* set, const WfParams* w, EventTimer* t, const PassArgs& a, uint64_t* launches) {
+    c = set;
+    W = w;
+    tt = t;
+    A = a;
+    b = cur = known_b = 0;
+    known_n = A.n_paths;
+    running = false;
+    tag0 = c->seen_tag;
+    c->seen_tag += (uint32_t)W->max_bounces + 1;
+    if ((size_t)A.n_paths > c->ps_cap) return fail(TPT_ERR_INTERNAL, "a pass holds more paths than were allocated");
+    if (W->max_bounces == 0) {
+      HIPC(wf_launch_clear_radiance(*W, A.n_paths, c->stream));
+      return TPT_OK;
+    }
+    if (A.n_paths <= TPT_WF_TAIL_FIRST) {
+      HIPC(wf_launch_tail(*W, cur, &A, A.n_paths, c->stream));
+      return TPT_OK;
+    }
+    const int rc = extend(&A, PathCount{nullptr, 0, 0}, launches);
+    return rc ? rc : shade(&A, launches);
+  }
+  // Queues the next bounce if its path count has been reported, or if the bounce before it had so
+  // many paths that it can be taken for more than a tail.
+  int poll(uint64_t* launches) {
+    if (!running) return TPT_OK;
+    const uint64_t got = __atomic_load_n(c->seen, __ATOMIC_ACQUIRE);
+    const uint32_t at = (uint32_t)(got >> 32) - tag0;  // the bounce reported last, if one of this pass's
+    if (at >= 1 && at <= (uint32_t)b) {
+      known_b = (int)at;
+      known_n = (uint32_t)got;
+    }
+    if (known_b == b) {
+      if (known_n > TPT_WF_TAIL_MAX) return shade(nullptr, launches);
+      running = false;
+      if (known_n > 0) HIPC(wf_launch_tail(*W, cur, nullptr, known_n, c->stream));
+      return TPT_OK;
+    }
+    if (known_b == b - 1 && known_n >= TPT_WF_AHEAD_MIN) return shade(nullptr, launches);
+    // A report leaves its kernels' run to act on it: a long wait means long kernels, and then the
+    // host need not spin.
+    if (++polls > 2000) std::this_thread::sleep_for(std::chrono::microseconds(20));
+    if (polls % 4096 == 0) {  // a stream that has stopped reports nothing more
+      const hipError_t e = hipStreamQuery(c->stream);
+      if (e != hipErrorNotReady && __atomic_load_n(c->seen, __ATOMIC_ACQUIRE) == got)
+        return fail(TPT_ERR_DEVICE, std::string("a bounce did not report its paths: ") + hipGetErrorString(e));
+    }
+    return TPT_OK;
+  }
+};
+
+// Runs `n` passes, pass i on path set i % nsets, each set's passes one after the other; begin(i)
+// describes a pass, finish(i) queues its accumulation and is called in order.
+template <class Begin, class Finish>
+int run_passes(tpt_ctx* c, const WfParams* W, EventTimer* const* tt, int nsets, uint64_t n, uint64_t* launches, Begin begin,
+               Finish finish) {
+  PassRun run[2];
+  uint64_t started = 0, finished = 0;
+  while (finished < n) {
+    while (started < n && started < finished + (uint64_t)nsets) {
+      const int j = (int)(started % (uint64_t)nsets);
+      const int rc = run[j].start(&c->set[j], &W[j], tt[j], begin(started), launches);
+      if (rc) return rc;
+      started++;
+    }
+    for (int j = 0; j < nsets; j++) {
+      const int rc = run[j].poll(launches);
+      if (rc) return rc;
+    }
+    while (finished < started && !run[finished % (uint64_t)nsets].running) {
+      const int rc = finish(finished);
+      if (rc) return rc;
+      finished++;
+    }
   }
   return TPT_OK;
 }
@@ -669,24 +774,25 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
     HIPC(hipStreamWaitEvent(c->set[1].stream, c->set[0].done, 0));
   }
   if (!adaptive) {
-    uint64_t pass = 0;
-    for (uint32_t p0 = 0; p0 < npix; p0 += pix_chunk) {
-      uint32_t np = std::min(pix_chunk, npix - p0);
-      for (uint32_t s0 = 0; s0 < spp; s0 += k) {
-        const int j = nsets == 2 ? (int)(pass & 1) : 0;
-        PathSet* S = &c->set[j];
-        uint32_t kk = std::min(k, spp - s0);
-        PassArgs A{np * kk, np, kk, p0, s0, nullptr, nullptr, pix_map};
-        rc = wf_bounces(S, W[j], A, *tt[j], &launches);
-        if (rc) return rc;
-        AccumArgs B{np, p0, kk, acc, acc_w, acc_sq};
-        // after the previous pass's accumulation (queued on the other set's stream)
-        if (nsets == 2 && pass > 0) HIPC(hipStreamWaitEvent(S->stream, c->set[j ^ 1].done, 0));
-        HIPC(wf_launch_accumulate(W[j], B, S->stream));
-        if (nsets == 2) HIPC(hipEventRecord(S->done, S->stream));
-        pass++;
-      }
-    }
+    const uint32_t groups = spp > 0 ? (spp + k - 1) / k : 0;  // sample groups of each pixel chunk
+    const uint64_t passes = (uint64_t)((npix + pix_chunk - 1) / pix_chunk) * groups;
+    auto pass_args = [&](uint64_t pass) {
+      const uint32_t p0 = (uint32_t)(pass / groups) * pix_chunk, s0 = (uint32_t)(pass % groups) * k;
+      const uint32_t np = std::min(pix_chunk, npix - p0), kk = std::min(k, spp - s0);
+      return PassArgs{np * kk, np, kk, p0, s0, nullptr, nullptr, pix_map};
+    };
+    rc = run_passes(c, W, tt, nsets, passes, &launches, pass_args, [&](uint64_t pass) -> int {
+      const int j = (int)(pass % (uint64_t)nsets);
+      PathSet* S = &c->set[j];
+      const PassArgs A = pass_args(pass);
+      AccumArgs B{A.n_pixels, A.pixel0, A.k, acc, acc_w, acc_sq};
+      // after the previous pass's accumulation (queued on the other set's stream)
+      if (nsets == 2 && pass > 0) HIPC(hipStreamWaitEvent(S->stream, c->set[j ^ 1].done, 0));
+      HIPC(wf_launch_accumulate(W[j], B, S->stream));
+      if (nsets == 2) HIPC(hipEventRecord(S->done, S->stream));
+      return TPT_OK;
+    });
+    if (rc) return rc;
     if (nsets == 2) HIPC(hipStreamWaitEvent(s, c->set[1].done, 0));
   } else {
     // render.rs:143-179 per pixel; each pass gives every active pixel k more samples
@@ -716,17 +822,20 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
       HIPC(hipStreamWaitEvent(c->set[1].stream, c->set[0].done, 0));
       // the active list in chunks of at most P / kk pixels, alternating between the sets (a
       // pixel's samples do not depend on its chunk or its position in the list)
-      int j = 0;
-      for (uint32_t c0 = 0; c0 < n_active; c0 += chunk, j ^= 1) {
-        PathSet* S = &c->set[j];
-        const uint32_t nc = std::min(chunk, n_active - c0);
-        PassArgs A{nc * kk, nc, kk, 0, 0, act_in + c0, c->nsamp.as<uint32_t>(), pix_map};
-        rc = wf_bounces(S, W[j], A, *tt[j], &launches);
-        if (rc) return rc;
-        AdaptiveArgs B{nc, kk, min_spp, spp, cfg->adaptive_threshold, act_in + c0, act_out, n_out,
+      const uint64_t chunks = (n_active + chunk - 1) / chunk;
+      auto pass_args = [&](uint64_t i) {
+        const uint32_t c0 = (uint32_t)i * chunk, nc = std::min(chunk, n_active - c0);
+        return PassArgs{nc * kk, nc, kk, 0, 0, act_in + c0, c->nsamp.as<uint32_t>(), pix_map};
+      };
+      rc = run_passes(c, W, tt, nsets, chunks, &launches, pass_args, [&](uint64_t i) -> int {
+        const int j = (int)(i % (uint64_t)nsets);
+        const PassArgs A = pass_args(i);
+        AdaptiveArgs B{A.n_pixels, kk, min_spp, spp, cfg->adaptive_threshold, A.active, act_out, n_out,
                        c->nsamp.as<uint32_t>(), c->welford.as<double>(), acc, acc_w, acc_sq};
-        HIPC(wf_launch_accumulate_adaptive(W[j], B, S->stream));
-      }
+        HIPC(wf_launch_accumulate_adaptive(W[j], B, c->set[j].stream));
+        return TPT_OK;
+      });
+      if (rc) return rc;
       HIPC(hipEventRecord(c->set[1].done, c->set[1].stream));
       HIPC(hipStreamWaitEvent(s, c->set[1].done, 0));
       HIPC(hipMemcpyAsync(&n_active, n_out, 4, hipMemcpyDeviceToHost, s));
@@ -737,7 +846,7 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
   }
   HIPC(total.mark());
   HIPC(hipStreamSynchronize(s));
-  uint64_t h[5] = {0, 0, 0, 0, 0};
+  uint64_t h[6] = {0, 0, 0, 0, 0, 0};
   for (int j = 0; j < nsets; j++) {
     uint32_t overflow = 0;
     HIPC(hipMemcpy(&overflow, W[j].ps.counters + TPT_CNT_OVERFLOW, 4, hipMemcpyDeviceToHost));
@@ -746,7 +855,7 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
       std::vector<uint64_t> seg(TPT_STAT_WORDS);
       HIPC(hipMemcpy(seg.data(), W[j].ps.stats, TPT_STAT_WORDS * 8, hipMemcpyDeviceToHost));
       for (int g = 0; g < TPT_WF_SEGS; g++)
-        for (int q = 0; q < 5; q++) h[q] += seg[(size_t)g * TPT_STAT_STRIDE + q];
+        for (int q = 0; q < 6; q++) h[q] += seg[(size_t)g * TPT_STAT_STRIDE + q];
     }
   }
   if (st) {
@@ -756,7 +865,7 @@ int render_wavefront(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* c
     st->elapsed_ms = total.pairs_ms();
     st->trace_kernel_ms = tt0.pairs_ms() + tt1.pairs_ms();
     st->trace_launches = launches;
-    st->trace_rays = h[0];
+    st->trace_rays = h[0] - h[5];
     st->light_samples = h[3];
     st->light_self_occluded = h[4];
   }

@@ -82,9 +82,23 @@ __device__ __forceinline__ void gen_path(const WfParams& W, const PassArgs& A, u
   camera_ray32(W.cam, x, y, W.inv_w, W.inv_h, *rng, o, d);
 }
 
+// Rays each wave takes at once: all 64 lanes while n rays fill the launched waves, else n spread
+// over the waves (at least TPT_WF_MIN_LANES each).
+__device__ __forceinline__ uint32_t lanes_per_wave(uint32_t n) {
+  const uint32_t waves = gridDim.x * (TPT_WF_BLOCK / 64), q = (n + waves - 1) / waves;
+  return max(min(q, 64u), (uint32_t)TPT_WF_MIN_LANES);
+}
+
 // A pass without bounces (max_bounces 0) gathers no radiance: clear its paths' sums.
 __global__ void __launch_bounds__(TPT_WF_BLOCK) k_clear_radiance(WfParams W, uint32_t n) {
   for (uint32_t i = gtid(); i < n; i += gridDim.x * blockDim.x) W.ps.L[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+__device__ __forceinline__ void tell_count(const WfParams& W, const PathCount& c) {
+  if (gtid() != 0 || !c.seen) return;
+  uint32_t n = 0;
+  for (int g = 0; g < TPT_WF_SEGS; g++) n += W.ps.counters[TPT_CNT_IDX(c.queue ? TPT_CNT_Q1 : TPT_CNT_Q0, g)];
+  __hip_atomic_store(c.seen, (uint64_t)c.tag << 32 | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // OVF: the scene's stack bound exceeds the LDS part, so the traversal stack may overflow to the
@@ -94,7 +108,7 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_clear_radiance(WfParams W, uin
 // code needs more); the traversal is VALU-bound, and more waves hide its load latency.
 template <bool OVF, bool GEN>
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(GEN ? 5 : 6)))
-k_extend(WfParams W, int cur, PassArgs A) {
+k_extend(WfParams W, int cur, PassArgs A, PathCount count) {
   __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
   QueueMap qm;
   uint32_t n;
@@ -115,6 +129,7 @@ k_extend(WfParams W, int cur, PassArgs A) {
     W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
   }
   if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
+  if (!GEN) tell_count(W, count);
   if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
   for (uint32_t i = gtid(); i < n; i += gridDim.x * blockDim.x) {
     f3 o, d;
@@ -137,8 +152,8 @@ k_extend(WfParams W, int cur, PassArgs A) {
 // step) and, once fewer than T lanes are still tracing (W.refill, or W.refill_first on the first
 // bounce), hands its idle lanes the next rays of the queue (one atomic per refill on a global
 // cursor; dynamic ray fetch, Aila and Laine 2009).  The hits are those of k_extend: each ray's traversal is the same sequence of steps.
-// The cursor (TPT_CNT_FETCH) is zero at launch: the render clears it, and every k_shade launch
-// clears it for the next extension launch.  Every wave exits once the cursor has passed the
+// The cursor (TPT_CNT_FETCH) is zero at launch: the render clears it, and every k_shade and
+// k_accumulate launch clears it for the next extension launch.  Every wave exits once the cursor has passed the
 // queue's end and its lanes are idle.  With the overflow path the resumable state needs more
 // registers: five waves per SIMD (96 VGPRs) for the later bounces and four (117) for the first
 // keep it out of scratch, where six and five spilled 44 and 64 bytes per lane that the loop
@@ -146,7 +161,7 @@ k_extend(WfParams W, int cur, PassArgs A) {
 // faster).
 template <bool OVF, bool GEN>
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(GEN && OVF ? 4 : GEN || OVF ? 5 : 6)))
-k_extend_refill(WfParams W, int cur, PassArgs A) {
+k_extend_refill(WfParams W, int cur, PassArgs A, PathCount count) {
   __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
   QueueMap qm;
   uint32_t n;
@@ -167,6 +182,7 @@ k_extend_refill(WfParams W, int cur, PassArgs A) {
     W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
   }
   if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
+  if (!GEN) tell_count(W, count);
   if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
   uint32_t* cursor = W.ps.counters + TPT_CNT_FETCH;
   const uint32_t lane = __lane_id();
@@ -214,10 +230,138 @@ __device__ __forceinline__ void add_radiance(float4* L, int32_t id, f3 c) {
   L[id] = make_float4(l.x + c.x, l.y + c.y, l.z + c.z, 0.f);
 }
 
-// ENV_NEE: the environment is an image with a non-zero texel, so environment NEE runs (the
-// variant without it needs fewer registers).  GEN: the first bounce; path i (position i) is
-// regenerated from its pixel and sample, as k_extend traced it, and its radiance sum L[i] is
-// written rather than added to.
+// One vertex of a path: its ray, throughput and random stream before shading; scatter() replaces
+// them by the next vertex's.
+struct PathVertex {
+  f3 o, d, beta;
+  float last_pdf;
+  uint32_t flags;  // bits 0-7 bounce, bit 8 last bounce non-delta
+  RngF32 rng{1};
+  __device__ __forceinline__ int bounce() const { return (int)(flags & 0xffu); }
+};
+// The surface a vertex scatters from.
+struct VertexSurface {
+  f3 p, ng;
+  int kind;
+  float4 mp;
+  float t;
+};
+// Shadow rays of a vertex and what they add to the path if they are unoccluded.
+struct VertexNee {
+  bool env, light;
+  f3 env_o, env_d, env_c;
+  f3 l_d, l_c;  // the shadow kernel rebuilds the light ray's origin p + eps wi and tmax
+  float l_dist;
+  uint64_t l_state;  // random stream before the light sample (for the self-occlusion decision)
+};
+
+// Miss, Russian roulette, emission and next-event estimation at hit h (integrator.rs:71-213);
+// false when the path ends here.  gather(c) receives the vertex's own radiance.  ENV_NEE: the
+// environment is an image with a non-zero texel, so environment NEE runs.
+template <bool ENV_NEE, class Gather>
+__device__ __forceinline__ bool shade_vertex(const WfParams& W, const HitRec& h, PathVertex& v, VertexSurface& sf,
+                                             VertexNee& nee, Gather gather) {
+  if (h.inst == -1) {
+    // miss (integrator.rs:71-83); a black map adds nothing, so its paths just end
+    if (!W.env.black) {
+      f3 bg = W.env.kind == TPT_ENV_IMAGE ? env_lookup32(W.env, v.d) : sky32(v.d);
+      f3 c = had(v.beta, bg);
+      if (W.env.kind == TPT_ENV_IMAGE && (v.flags & 0x100u)) c = c * mis_weight(v.last_pdf, env_pdf32(W.env, v.d));
+      gather(clamp_luminance(c, (float)TPT_FIREFLY_CLAMP));
+    }
+    return false;
+  }
+  if (v.bounce() >= W.rr_start) {  // integrator.rs:89-95
+    float q = fmaxf(fminf(fmaxf(fmaxf(v.beta.x, v.beta.y), v.beta.z), 0.95f), 0.05f);
+    if (v.rng.uni() > q) return false;
+    v.beta = v.beta / q;
+  }
+  int mat;
+  sf.t = __int_as_float(h.t);
+  hit_geometry32(W.S, h.inst, h.prim, sf.t, v.o, v.d, &sf.p, &sf.ng, &mat);
+  sf.kind = W.mats.kind[mat];
+  sf.mp = W.mats.p32[mat];
+  const f3 mc = f3of(sf.mp), p = sf.p;
+  if (sf.kind == TPT_MAT_DIFFUSE_LIGHT) {  // integrator.rs:100-104
+    gather(clamp_luminance(had(v.beta, mc), (float)TPT_FIREFLY_CLAMP));
+    return false;
+  }
+  if (mat_is_delta(sf.kind)) return true;
+  f3 n_o = dot(sf.ng, v.d) < 0.f ? sf.ng : -sf.ng;  // oriented_normal (integrator.rs:138-140)
+  f3 wo = vnorm(-v.d);
+  // nee_environment (integrator.rs:148-172); a black map contributes nothing, so the
+  // FP32 form skips it (its own random streams need not follow the reference's draws)
+  if (ENV_NEE) {
+    f3 wi, li;
+    float pdf_env;
+    env_sample32(W.env, v.rng, &wi, &li, &pdf_env);
+    float cs = fmaxf(dot(n_o, wi), 0.f);
+    if (cs > 0.f && pdf_env > 0.f && (li.x != 0.f || li.y != 0.f || li.z != 0.f)) {
+      f3 f;
+      float pdf_b;
+      bsdf_eval(sf.kind, mc, sf.mp.w, wo, wi, n_o, &f, &pdf_b);
+      f3 c = had(had(v.beta, f), li) * (cs * mis_weight(pdf_env, pdf_b) / pdf_env);
+      if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
+        nee.env_o = p + (float)TPT_RAY_EPSILON * wi;
+        nee.env_d = wi;
+        nee.env_c = c;
+        nee.env = true;
+      }
+    }
+  }
+  LightSample32 ls;  // nee_area_light (integrator.rs:178-213)
+  const uint64_t light_state = v.rng.p.state;
+  if (sample_light32(W.lights, v.rng, p, &ls)) {
+    f3 to_light = ls.pos - p;
+    float dist = sqrtf(dot(to_light, to_light));
+    if (dist > 1e-6f) {
+      f3 wi = to_light / dist;
+      float cs = fmaxf(dot(n_o, wi), 0.f);
+      if (cs > 0.f) {
+        f3 f;
+        float pdf_b;
+        bsdf_eval(sf.kind, mc, sf.mp.w, wo, wi, n_o, &f, &pdf_b);
+        f3 c = had(had(v.beta, f), ls.emit) * (cs * mis_weight(ls.pdf, pdf_b) / ls.pdf);
+        if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
+          nee.l_d = wi;
+          nee.l_c = c;
+          nee.l_dist = dist;
+          nee.l_state = light_state;
+          nee.light = true;
+        }
+      }
+    }
+  }
+  return true;
+}
+
+// BSDF sampling: v becomes the next vertex's ray; false when the path ends.
+__device__ __forceinline__ bool scatter_vertex(const WfParams& W, const VertexSurface& sf, PathVertex& v) {
+  if (v.bounce() + 1 >= W.max_bounces) return false;  // the scattered ray of the last bounce is never traced
+  BsdfSample<float> bs;
+  if (!bsdf_sample(sf.kind, f3of(sf.mp), sf.mp.w, v.d, sf.p, sf.ng, sf.t, v.rng, &bs)) return false;
+  v.beta = had(v.beta, bs.weight);
+  v.o = bs.o;
+  v.d = bs.d;
+  v.last_pdf = bs.pdf;
+  v.flags = (uint32_t)(v.bounce() + 1) | (bs.is_delta ? 0u : 0x100u);
+  return true;
+}
+
+__device__ __forceinline__ void load_vertex(const PathState& ps, int cur, uint32_t slot, PathVertex* v, int32_t* id) {
+  const float4 o4 = ps.o[cur][slot], d4 = ps.d[cur][slot], b4 = ps.beta[cur][slot];
+  v->o = f3of(o4);
+  v->d = f3of(d4);
+  v->beta = f3of(b4);
+  *id = __float_as_int(b4.w);
+  v->last_pdf = o4.w;
+  v->flags = __float_as_uint(d4.w);
+  v->rng.p.state = ps.rng[cur][slot];
+}
+
+// ENV_NEE: see shade_vertex (the variant without it needs fewer registers).  GEN: the first
+// bounce; path i (position i) is regenerated from its pixel and sample, as k_extend traced it,
+// and its radiance sum L[i] is written rather than added to.
 template <bool ENV_NEE, bool GEN>
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_shade(WfParams W, int cur, PassArgs A) {
@@ -235,32 +379,22 @@ k_shade(WfParams W, int cur, PassArgs A) {
   if (gtid() == 0) W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next extension launch (k_extend_refill)
   for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
     const uint32_t i = base + threadIdx.x;
-    bool alive = false, has_env = false, has_light = false;
     // path state (valid when i < n)
-    f3 o = mk(0.f, 0.f, 0.f), d = o, beta = o;
-    float last_pdf = 0.f;
-    uint32_t flags = 0;
+    PathVertex v;
+    v.o = v.d = v.beta = mk(0.f, 0.f, 0.f);
+    v.last_pdf = 0.f;
+    v.flags = 0;
     int32_t id = 0;
-    RngF32 rng(1);
-    int4 h4 = make_int4(0, -1, 0, 0);
+    HitRec h{0, -1, 0};
     if (i < n) {
       if constexpr (GEN) {
-        gen_path(W, A, i, &rng, &o, &d);
-        beta = mk(1.f, 1.f, 1.f);
+        gen_path(W, A, i, &v.rng, &v.o, &v.d);
+        v.beta = mk(1.f, 1.f, 1.f);
         id = (int32_t)i;
       } else {
-        const uint32_t slot = qm.slot(i);
-        float4 o4 = W.ps.o[cur][slot], d4 = W.ps.d[cur][slot], b4 = W.ps.beta[cur][slot];
-        o = f3of(o4);
-        d = f3of(d4);
-        beta = f3of(b4);
-        id = __float_as_int(b4.w);
-        last_pdf = o4.w;
-        flags = __float_as_uint(d4.w);
-        rng.p.state = W.ps.rng[cur][slot];
+        load_vertex(W.ps, cur, qm.slot(i), &v, &id);
       }
-      const HitRec hr = W.ps.hit[i];
-      h4 = make_int4(hr.t, hr.inst, hr.prim, 0);
+      h = W.ps.hit[i];
     }
     // radiance of this bounce: added to L[id], or (first bounce) gathered and written once
     f3 l0 = mk(0.f, 0.f, 0.f);
@@ -268,127 +402,40 @@ k_shade(WfParams W, int cur, PassArgs A) {
       if constexpr (GEN) l0 = l0 + c;
       else add_radiance(W.ps.L, id, c);
     };
-    const int bounce = (int)(flags & 0xffu);
-    const bool last_nd = (flags & 0x100u) != 0;
-    // ---- phase 1: miss, Russian roulette, emission, next-event estimation
-    float4 sh_c0 = make_float4(0.f, 0.f, 0.f, 0.f), sh_c1 = sh_c0;
-    float4 sh_o0 = sh_c0, sh_d0 = sh_c0, sh_d1 = sh_c0, sh_l = sh_c0;  // 0: environment, 1: light
-    uint64_t sh_lv = 0;
-    bool go = false;  // hit a scattering surface: sample the BSDF in phase 2
-    f3 p = mk(0.f, 0.f, 0.f), ng = p;
-    int mat = 0, kind = 0;
-    float4 mp = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < n) {
-      if (h4.y == -1) {
-        // miss (integrator.rs:71-83); a black map adds nothing, so its paths just end
-        if (!W.env.black) {
-          f3 bg = W.env.kind == TPT_ENV_IMAGE ? env_lookup32(W.env, d) : sky32(d);
-          f3 c = had(beta, bg);
-          if (W.env.kind == TPT_ENV_IMAGE && last_nd) c = c * mis_weight(last_pdf, env_pdf32(W.env, d));
-          gather(clamp_luminance(c, (float)TPT_FIREFLY_CLAMP));
-        }
-      } else {
-        go = true;
-        if (bounce >= W.rr_start) {  // integrator.rs:89-95
-          float q = fmaxf(fminf(fmaxf(fmaxf(beta.x, beta.y), beta.z), 0.95f), 0.05f);
-          if (rng.uni() > q) go = false;
-          else beta = beta / q;
-        }
-        if (go) {
-          const float t = __int_as_float(h4.x);
-          hit_geometry32(W.S, h4.y, h4.z, t, o, d, &p, &ng, &mat);
-          kind = W.mats.kind[mat];
-          mp = W.mats.p32[mat];
-          const f3 mc = f3of(mp);
-          if (kind == TPT_MAT_DIFFUSE_LIGHT) {  // integrator.rs:100-104
-            gather(clamp_luminance(had(beta, mc), (float)TPT_FIREFLY_CLAMP));
-            go = false;
-          } else if (!mat_is_delta(kind)) {
-            f3 n_o = dot(ng, d) < 0.f ? ng : -ng;  // oriented_normal (integrator.rs:138-140)
-            f3 wo = vnorm(-d);
-            // nee_environment (integrator.rs:148-172); a black map contributes nothing, so the
-            // FP32 form skips it (its own random streams need not follow the reference's draws)
-            if (ENV_NEE) {
-              f3 wi, li;
-              float pdf_env;
-              env_sample32(W.env, rng, &wi, &li, &pdf_env);
-              float cs = fmaxf(dot(n_o, wi), 0.f);
-              if (cs > 0.f && pdf_env > 0.f && (li.x != 0.f || li.y != 0.f || li.z != 0.f)) {
-                f3 f;
-                float pdf_b;
-                bsdf_eval(kind, mc, mp.w, wo, wi, n_o, &f, &pdf_b);
-                f3 c = had(had(beta, f), li) * (cs * mis_weight(pdf_env, pdf_b) / pdf_env);
-                if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
-                  f3 so = p + (float)TPT_RAY_EPSILON * wi;
-                  sh_o0 = make_float4(so.x, so.y, so.z, 1e30f);
-                  sh_d0 = make_float4(wi.x, wi.y, wi.z, __int_as_float(id));
-                  sh_c0 = make_float4(c.x, c.y, c.z, 1.f);
-                  has_env = true;
-                }
-              }
-            }
-            LightSample32 ls;  // nee_area_light (integrator.rs:178-213)
-            const uint64_t light_state = rng.p.state;
-            if (sample_light32(W.lights, rng, p, &ls)) {
-              f3 to_light = ls.pos - p;
-              float dist = sqrtf(dot(to_light, to_light));
-              if (dist > 1e-6f) {
-                f3 wi = to_light / dist;
-                float cs = fmaxf(dot(n_o, wi), 0.f);
-                if (cs > 0.f) {
-                  f3 f;
-                  float pdf_b;
-                  bsdf_eval(kind, mc, mp.w, wo, wi, n_o, &f, &pdf_b);
-                  f3 c = had(had(beta, f), ls.emit) * (cs * mis_weight(ls.pdf, pdf_b) / ls.pdf);
-                  if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
-                    // the shadow kernel rebuilds origin p + eps wi and tmax from p and dist
-                    sh_d1 = make_float4(wi.x, wi.y, wi.z, __int_as_float(id));
-                    sh_c1 = make_float4(c.x, c.y, c.z, dist);
-                    sh_l = make_float4(p.x, p.y, p.z, __int_as_float((int32_t)i));  // also for k_light_selfocc
-                    sh_lv = light_state;
-                    has_light = true;
-                  }
-                }
-              }
-            }
-          }
-        }
-      }
-    }
+    VertexSurface sf;
+    sf.p = sf.ng = mk(0.f, 0.f, 0.f);
+    sf.kind = 0;
+    sf.mp = make_float4(0.f, 0.f, 0.f, 0.f);
+    sf.t = 0.f;
+    VertexNee nee;
+    nee.env = nee.light = false;
+    nee.env_o = nee.env_d = nee.env_c = nee.l_d = nee.l_c = mk(0.f, 0.f, 0.f);
+    nee.l_dist = 0.f;
+    nee.l_state = 0;
+    bool go = false;  // hit a scattering surface: sample the BSDF
+    if (i < n) go = shade_vertex<ENV_NEE>(W, h, v, sf, nee, gather);
     if (GEN && i < n) W.ps.L[id] = make_float4(l0.x, l0.y, l0.z, 0.f);
-    const uint32_t je = ENV_NEE ? seg_slot(has_env, W.ps, TPT_CNT_SH, s_slot) : UINT32_MAX;
-    if (ENV_NEE && has_env && je != UINT32_MAX) {
-      W.ps.sh_o[0][je] = sh_o0;
-      W.ps.sh_d[0][je] = sh_d0;
-      W.ps.sh_c[0][je] = sh_c0;
+    const uint32_t je = ENV_NEE ? seg_slot(nee.env, W.ps, TPT_CNT_SH, s_slot) : UINT32_MAX;
+    if (ENV_NEE && nee.env && je != UINT32_MAX) {
+      W.ps.sh_o[0][je] = make_float4(nee.env_o.x, nee.env_o.y, nee.env_o.z, 1e30f);
+      W.ps.sh_d[0][je] = make_float4(nee.env_d.x, nee.env_d.y, nee.env_d.z, __int_as_float(id));
+      W.ps.sh_c[0][je] = make_float4(nee.env_c.x, nee.env_c.y, nee.env_c.z, 1.f);
     }
-    const uint32_t jl = seg_slot(has_light, W.ps, TPT_CNT_SHL, s_slot);
-    if (has_light && jl != UINT32_MAX) {
-      W.ps.sh_d[1][jl] = sh_d1;
-      W.ps.sh_c[1][jl] = sh_c1;
-      W.ps.sh_l[jl] = sh_l;
-      W.ps.sh_lv[jl] = sh_lv;
+    const uint32_t jl = seg_slot(nee.light, W.ps, TPT_CNT_SHL, s_slot);
+    if (nee.light && jl != UINT32_MAX) {
+      W.ps.sh_d[1][jl] = make_float4(nee.l_d.x, nee.l_d.y, nee.l_d.z, __int_as_float(id));
+      W.ps.sh_c[1][jl] = make_float4(nee.l_c.x, nee.l_c.y, nee.l_c.z, nee.l_dist);
+      W.ps.sh_l[jl] = make_float4(sf.p.x, sf.p.y, sf.p.z, __int_as_float((int32_t)i));  // also for k_light_selfocc
+      W.ps.sh_lv[jl] = nee.l_state;
     }
-    // ---- phase 2: BSDF sampling; survivors go densely into the next buffer set
-    bool bsdf_nd = false;
-    if (go && bounce + 1 < W.max_bounces) {  // the scattered ray of the last bounce is never traced
-      BsdfSample<float> bs;
-      if (bsdf_sample(kind, f3of(mp), mp.w, d, p, ng, __int_as_float(h4.x), rng, &bs)) {
-        beta = had(beta, bs.weight);
-        o = bs.o;
-        d = bs.d;
-        last_pdf = bs.pdf;
-        bsdf_nd = !bs.is_delta;
-        alive = true;
-      }
-    }
+    // BSDF sampling; survivors go densely into the next buffer set
+    const bool alive = go && scatter_vertex(W, sf, v);
     const uint32_t k = seg_slot(alive, W.ps, cur ? TPT_CNT_Q0 : TPT_CNT_Q1, s_slot);
     if (alive && k != UINT32_MAX) {
-      uint32_t nflags = (uint32_t)(bounce + 1) | (bsdf_nd ? 0x100u : 0u);
-      W.ps.o[nxt][k] = make_float4(o.x, o.y, o.z, last_pdf);
-      W.ps.d[nxt][k] = make_float4(d.x, d.y, d.z, __uint_as_float(nflags));
-      W.ps.beta[nxt][k] = make_float4(beta.x, beta.y, beta.z, __int_as_float(id));
-      W.ps.rng[nxt][k] = rng.p.state;
+      W.ps.o[nxt][k] = make_float4(v.o.x, v.o.y, v.o.z, v.last_pdf);
+      W.ps.d[nxt][k] = make_float4(v.d.x, v.d.y, v.d.z, __uint_as_float(v.flags));
+      W.ps.beta[nxt][k] = make_float4(v.beta.x, v.beta.y, v.beta.z, __int_as_float(id));
+      W.ps.rng[nxt][k] = v.rng.p.state;
     }
   }
 }
@@ -402,8 +449,10 @@ k_shade(WfParams W, int cur, PassArgs A) {
 // remain go densely into the SHK queue, so k_shadow's waves carry no lanes for dropped rays
 // (about 30% on a rectangle light).
 template <bool GEN>
-__global__ void __launch_bounds__(TPT_WF_BLOCK) k_light_selfocc(WfParams W, int cur, PassArgs A) {
+__global__ void __launch_bounds__(TPT_WF_BLOCK) k_light_selfocc(WfParams W, int cur, PassArgs A,
+                                                                 PathCount count) {
   __shared__ uint32_t s_slot[8];
+  tell_count(W, count);
   QueueMap qm, qp;
   qm.load(W.ps.counters, TPT_CNT_SHL, W.ps.seg_cap);
   if constexpr (!GEN) qp.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
@@ -449,7 +498,8 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_light_selfocc(WfParams W, int 
 // contribution to its path's radiance.  A path has at most one ray per queue, so the
 // read-modify-write of L[id] has a single writer per launch.
 template <bool OVF>
-__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_shadow(WfParams W, int queue) {
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_shadow(WfParams W, int queue, PathCount count) {
+  tell_count(W, count);
   __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
   QueueMap qm;
   qm.load(W.ps.counters, queue ? TPT_CNT_SHK : TPT_CNT_SH, W.ps.seg_cap);
@@ -482,6 +532,105 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_
               (unsigned long long)tot);
 }
 
+// The rest of a few paths in one launch: each lane walks its path to the end -- extension, shading,
+// the light self-occlusion decision, shadow rays and scattering by the same functions as the
+// kernels above, contributions added in their order, so a path's radiance is the same bit for bit.
+// GEN: the whole paths of a small pass (camera rays generated here); otherwise the paths of queue
+// cur, whose hits this bounce's extension has stored.
+template <bool OVF, bool ENV_NEE, bool GEN>
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
+k_tail(WfParams W, int cur, PassArgs A) {
+  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
+  QueueMap qm;
+  uint32_t n;
+  if constexpr (GEN) {
+    n = A.n_paths;
+  } else {
+    qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
+    n = qm.n;
+  }
+  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
+                     TPT_WF_STACK};
+  const uint32_t lanes = lanes_per_wave(n);
+  uint32_t next = (gtid() >> 6) * lanes + __lane_id();
+  if (__lane_id() >= lanes) next = n;
+  uint32_t n_ext = 0, n_sh = 0, n_light = 0, n_drop = 0;
+  bool alive = false;
+  PathVertex v;
+  int32_t id = 0;
+  f3 L = mk(0.f, 0.f, 0.f);
+  for (;;) {
+    HitRec h;
+    bool have_hit = false;
+    if (!alive) {
+      if (next >= n) break;
+      if constexpr (GEN) {
+        gen_path(W, A, next, &v.rng, &v.o, &v.d);
+        v.beta = mk(1.f, 1.f, 1.f);
+        v.last_pdf = 0.f;
+        v.flags = 0;
+        id = (int32_t)next;
+        L = mk(0.f, 0.f, 0.f);
+      } else {
+        load_vertex(W.ps, cur, qm.slot(next), &v, &id);
+        h = W.ps.hit[next];
+        have_hit = true;
+        L = f3of(W.ps.L[id]);
+      }
+      next += gridDim.x * (TPT_WF_BLOCK / 64) * lanes;
+      alive = true;
+    }
+    if (!have_hit) {
+      HitF32 t;
+      trace_f32<false>(W.S, v.o, v.d, (float)TPT_RAY_EPSILON, 1e30f, &t, st);
+      h = HitRec{__float_as_int(t.t), t.inst, t.prim};
+      n_ext++;
+    }
+    VertexSurface sf;
+    VertexNee nee;
+    nee.env = nee.light = false;
+    alive = shade_vertex<ENV_NEE>(W, h, v, sf, nee, [&](f3 c) { L = L + c; });
+    if (nee.light) {  // k_light_selfocc, then k_shadow on the light queue
+      n_light++;
+      RngF32 rng(1);
+      rng.p.state = nee.l_state;
+      const int idx = light_pick32(W.lights, rng);
+      const double lu = rng.uni53(), lv = rng.uni53();
+      const D3 p64 = hit_point64(W.S64, W.S.tri_orig, h.inst, h.prim, v.o, v.d, sf.p);
+      if (light_self_occluded64(W.S64, W.lights, idx, p64, lu, lv)) {
+        n_drop++;
+      } else {
+        HitF32 t;
+        n_sh++;
+        if (!trace_f32<true>(W.S, sf.p + (float)TPT_RAY_EPSILON * nee.l_d, nee.l_d, (float)TPT_RAY_EPSILON,
+                             light_shadow_tmax32(nee.l_dist), &t, st))
+          L = L + nee.l_c;
+      }
+    }
+    if (ENV_NEE && nee.env) {  // k_shadow on the environment queue
+      HitF32 t;
+      n_sh++;
+      if (!trace_f32<true>(W.S, nee.env_o, nee.env_d, (float)TPT_RAY_EPSILON, 1e30f, &t, st)) L = L + nee.env_c;
+    }
+    alive = alive && scatter_vertex(W, sf, v);
+    if (!alive) W.ps.L[id] = make_float4(L.x, L.y, L.z, 0.f);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    n_ext += (uint32_t)__shfl_down((int)n_ext, off);
+    n_sh += (uint32_t)__shfl_down((int)n_sh, off);
+    n_light += (uint32_t)__shfl_down((int)n_light, off);
+    n_drop += (uint32_t)__shfl_down((int)n_drop, off);
+  }
+  if (__lane_id() == 0 && (n_ext | n_sh | n_light)) {
+    unsigned long long* stat = (unsigned long long*)W.ps.stats + (blockIdx.x & (TPT_WF_SEGS - 1)) * TPT_STAT_STRIDE;
+    atomicAdd(&stat[0], (unsigned long long)n_ext);
+    atomicAdd(&stat[1], (unsigned long long)n_sh);
+    atomicAdd(&stat[3], (unsigned long long)n_light);
+    atomicAdd(&stat[4], (unsigned long long)n_drop);
+    atomicAdd(&stat[5], (unsigned long long)n_ext);
+  }
+}
+
 // Non-adaptive: pixel p accumulates the k paths of this pass, in sample order.
 __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate(WfParams W, AccumArgs A) {
   for (uint32_t p = gtid(); p < A.n_pixels; p += gridDim.x * blockDim.x) {
@@ -499,7 +648,10 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate(WfParams W, AccumAr
     A.acc_w[g_pix] += (double)A.k;
     if (A.acc_sq) { A.acc_sq[3 * g_pix] += r2; A.acc_sq[3 * g_pix + 1] += g2; A.acc_sq[3 * g_pix + 2] += b2; }
   }
-  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[2], (unsigned long long)A.n_pixels * A.k);
+  if (gtid() == 0) {
+    W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next pass
+    atomicAdd((unsigned long long*)&W.ps.stats[2], (unsigned long long)A.n_pixels * A.k);
+  }
 }
 
 // Adaptive (render.rs:143-179): for each active pixel take its k new samples in sample order,
@@ -509,6 +661,7 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate_adaptive(WfParams W
   __shared__ uint32_t s_slot[8];
   const uint32_t stride = gridDim.x * blockDim.x;
   uint32_t kept = 0;  // samples this thread added to its pixels (the paths the render counts)
+  if (gtid() == 0) W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next pass
   for (uint32_t base = blockIdx.x * blockDim.x; base < A.n_active; base += stride) {
     uint32_t j = base + threadIdx.x;
     bool keep = false;
@@ -563,7 +716,8 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate_adaptive(WfParams W
 // cursor TPT_CNT_FETCH_SH(queue) is cleared by the extension kernel of the same bounce.
 template <bool OVF>
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
-k_shadow_refill(WfParams W, int queue) {
+k_shadow_refill(WfParams W, int queue, PathCount count) {
+  tell_count(W, count);
   __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
   QueueMap qm;
   qm.load(W.ps.counters, queue ? TPT_CNT_SHK : TPT_CNT_SH, W.ps.seg_cap);
@@ -661,44 +815,42 @@ hipError_t wf_launch_clear_radiance(const WfParams& W, uint32_t n, hipStream_t s
   hipLaunchKernelGGL(k_clear_radiance, dim3(grid_for(n)), dim3(TPT_WF_BLOCK), 0, s, W, n);
   return hipGetLastError();
 }
-// A launch, timed by events that the dispatch records itself when ev0 is given.
+// Extension launches, timed by events that the dispatch records itself when ev0 is given.
 template <class K>
-static void launch_timed(K kernel, dim3 grid, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, const WfParams& W, int cur,
-                         const PassArgs& A) {
-  if (ev0) hipExtLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, ev0, ev1, 0, W, cur, A);
-  else hipLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, W, cur, A);
+static void launch_timed(K kernel, uint32_t max_n, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, const WfParams& W,
+                         int cur, const PassArgs& A, const PathCount& count) {
+  const dim3 grid = grid_of(max_n, (const void*)kernel);
+  if (ev0) hipExtLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, ev0, ev1, 0, W, cur, A, count);
+  else hipLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, W, cur, A, count);
 }
-template <bool OVF, bool GEN>
-static void launch_extend(const WfParams& W, int cur, const PassArgs& A, uint32_t max_n, hipStream_t s, hipEvent_t ev0,
-                          hipEvent_t ev1) {
-  launch_timed(k_extend<OVF, GEN>, grid_of(max_n, (const void*)k_extend<OVF, GEN>), s, ev0, ev1, W, cur, A);
-}
-template <bool OVF, bool GEN>
-static void launch_extend_refill(const WfParams& W, int cur, const PassArgs& A, uint32_t max_n, hipStream_t s,
-                                 hipEvent_t ev0, hipEvent_t ev1) {
-  launch_timed(k_extend_refill<OVF, GEN>, grid_of(max_n, (const void*)k_extend_refill<OVF, GEN>), s, ev0, ev1, W, cur,
-               A);
-}
-hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s,
-                            hipEvent_t ev0, hipEvent_t ev1) {
+hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, const PathCount& count, uint32_t max_n,
+                            hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
   const PassArgs A = gen ? *gen : PassArgs{};
+  auto launch = [&](auto kernel) { launch_timed(kernel, max_n, s, ev0, ev1, W, cur, A, count); };
   if (gen ? W.refill_first > 0 : W.refill > 0) {
-    if (W.gstack) {
-      if (gen) launch_extend_refill<true, true>(W, cur, A, max_n, s, ev0, ev1);
-      else launch_extend_refill<true, false>(W, cur, A, max_n, s, ev0, ev1);
-    } else {
-      if (gen) launch_extend_refill<false, true>(W, cur, A, max_n, s, ev0, ev1);
-      else launch_extend_refill<false, false>(W, cur, A, max_n, s, ev0, ev1);
-    }
-    return hipGetLastError();
-  }
-  if (W.gstack) {
-    if (gen) launch_extend<true, true>(W, cur, A, max_n, s, ev0, ev1);
-    else launch_extend<true, false>(W, cur, A, max_n, s, ev0, ev1);
+    if (W.gstack) gen ? launch(k_extend_refill<true, true>) : launch(k_extend_refill<true, false>);
+    else gen ? launch(k_extend_refill<false, true>) : launch(k_extend_refill<false, false>);
   } else {
-    if (gen) launch_extend<false, true>(W, cur, A, max_n, s, ev0, ev1);
-    else launch_extend<false, false>(W, cur, A, max_n, s, ev0, ev1);
+    if (W.gstack) gen ? launch(k_extend<true, true>) : launch(k_extend<true, false>);
+    else gen ? launch(k_extend<false, true>) : launch(k_extend<false, false>);
   }
+  return hipGetLastError();
+}
+template <bool OVF, bool ENV_NEE>
+static void launch_tail(const WfParams& W, int cur, const PassArgs* gen, uint32_t n, hipStream_t s) {
+  const PassArgs A = gen ? *gen : PassArgs{};
+  auto launch = [&](auto kernel) {
+    const uint32_t waves = (n + TPT_WF_MIN_LANES - 1) / TPT_WF_MIN_LANES;
+    hipLaunchKernelGGL(kernel, grid_of(std::min(waves, 1u << 20) * 64, (const void*)kernel), dim3(TPT_WF_BLOCK), 0, s, W,
+                       cur, A);
+  };
+  if (gen) launch(k_tail<OVF, ENV_NEE, true>);
+  else launch(k_tail<OVF, ENV_NEE, false>);
+}
+static inline bool env_nee(const WfParams& W) { return W.env.kind == TPT_ENV_IMAGE && !W.env.black; }
+hipError_t wf_launch_tail(const WfParams& W, int cur, const PassArgs* gen, uint32_t n, hipStream_t s) {
+  if (W.gstack) env_nee(W) ? launch_tail<true, true>(W, cur, gen, n, s) : launch_tail<true, false>(W, cur, gen, n, s);
+  else env_nee(W) ? launch_tail<false, true>(W, cur, gen, n, s) : launch_tail<false, false>(W, cur, gen, n, s);
   return hipGetLastError();
 }
 template <bool ENV_NEE, bool GEN>
@@ -708,7 +860,7 @@ static void launch_shade(const WfParams& W, int cur, const PassArgs& A, uint32_t
 }
 hipError_t wf_launch_shade(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s) {
   const PassArgs A = gen ? *gen : PassArgs{};
-  if (W.env.kind == TPT_ENV_IMAGE && !W.env.black) {
+  if (env_nee(W)) {
     if (gen) launch_shade<true, true>(W, cur, A, max_n, s);
     else launch_shade<true, false>(W, cur, A, max_n, s);
   } else {
@@ -717,31 +869,21 @@ hipError_t wf_launch_shade(const WfParams& W, int cur, const PassArgs* gen, uint
   }
   return hipGetLastError();
 }
-hipError_t wf_launch_light_selfocc(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s) {
+hipError_t wf_launch_light_selfocc(const WfParams& W, int cur, const PassArgs* gen, const PathCount& count,
+                                   uint32_t max_n, hipStream_t s) {
   const PassArgs A = gen ? *gen : PassArgs{};
-  if (gen)
-    hipLaunchKernelGGL(k_light_selfocc<true>, grid_of(max_n, (const void*)k_light_selfocc<true>), dim3(TPT_WF_BLOCK), 0, s,
-                       W, cur, A);
-  else
-    hipLaunchKernelGGL(k_light_selfocc<false>, grid_of(max_n, (const void*)k_light_selfocc<false>), dim3(TPT_WF_BLOCK), 0,
-                       s, W, cur, A);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid_of(max_n, (const void*)kernel), dim3(TPT_WF_BLOCK), 0, s, W, cur, A, count);
+  };
+  gen ? launch(k_light_selfocc<true>) : launch(k_light_selfocc<false>);
   return hipGetLastError();
 }
-hipError_t wf_launch_shadow(const WfParams& W, int queue, uint32_t max_n, hipStream_t s) {
-  if (W.refill_sh > 0) {
-    if (W.gstack)
-      hipLaunchKernelGGL(k_shadow_refill<true>, grid_of(max_n, (const void*)k_shadow_refill<true>), dim3(TPT_WF_BLOCK),
-                         0, s, W, queue);
-    else
-      hipLaunchKernelGGL(k_shadow_refill<false>, grid_of(max_n, (const void*)k_shadow_refill<false>),
-                         dim3(TPT_WF_BLOCK), 0, s, W, queue);
-    return hipGetLastError();
-  }
-  if (W.gstack)
-    hipLaunchKernelGGL(k_shadow<true>, grid_of(max_n, (const void*)k_shadow<true>), dim3(TPT_WF_BLOCK), 0, s, W, queue);
-  else
-    hipLaunchKernelGGL(k_shadow<false>, grid_of(max_n, (const void*)k_shadow<false>), dim3(TPT_WF_BLOCK), 0, s, W,
-                       queue);
+hipError_t wf_launch_shadow(const WfParams& W, int queue, const PathCount& count, uint32_t max_n, hipStream_t s) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid_of(max_n, (const void*)kernel), dim3(TPT_WF_BLOCK), 0, s, W, queue, count);
+  };
+  if (W.refill_sh > 0) W.gstack ? launch(k_shadow_refill<true>) : launch(k_shadow_refill<false>);
+  else W.gstack ? launch(k_shadow<true>) : launch(k_shadow<false>);
   return hipGetLastError();
 }
 hipError_t wf_launch_accumulate(const WfParams& W, const AccumArgs& A, hipStream_t s) {
@@ -753,6 +895,8 @@ hipError_t wf_launch_accumulate_adaptive(const WfParams& W, const AdaptiveArgs& 
   return hipGetLastError();
 }
 // Upper bound of the threads of any launch above over n entries (sizes per-thread areas).
-uint32_t wf_grid_threads(uint32_t n) { return grid_for(n) * TPT_WF_BLOCK; }
+uint32_t wf_grid_threads(uint32_t n) {
+  return grid_for(std::min(n, 1u << 20) * (64 / TPT_WF_MIN_LANES)) * TPT_WF_BLOCK;
+}
 
 }  // namespace tpt

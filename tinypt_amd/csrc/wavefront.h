@@ -36,6 +36,22 @@ static_assert(TPT_WF_BLOCK % 64 == 0 && TPT_WF_BLOCK / 64 <= 7, "block_slot keep
 #define TPT_NUM_CNT (TPT_CNT_FETCH + 3 * TPT_CNT_STRIDE)
 #define TPT_STAT_STRIDE 32  // uint64 words of statistics per segment (256 B)
 #define TPT_STAT_WORDS (TPT_WF_SEGS * TPT_STAT_STRIDE)
+// Few paths: a bounce's four or five launches take 40 to 300 us however few paths they have (cold
+// instruction and scalar caches, the longest traversal of 64 divergent lanes), so k_tail walks the
+// last paths to their ends in one launch.  It takes a pass of at most TPT_WF_TAIL_FIRST paths whole
+// and the others once at most TPT_WF_TAIL_MAX paths are left.  Measured on MI355X, us per render,
+// bounce by bounce / with k_tail: Cornell box of 16K paths 654 / 241, 256K 756 / 445, 512K 842 / 645;
+// 20k-triangle mesh of 16K paths 1343 / 452, 256K 2017 / 1181; a whole pass of 1M paths is slower
+// (Cornell 1038 / 1098).  Left-over paths: the 1.31M-triangle
+// mesh at 1080p x 32 spp 43.0 / 39.5 ms, a 20k-triangle mesh of 3.6M paths 4.09 / 3.49 ms, each within
+// 1% for limits of 2^16 to 2^18.
+#define TPT_WF_TAIL_FIRST (1u << 18)
+#define TPT_WF_TAIL_MAX (1u << 17)
+// A bounce is queued before its path count is known if the bounce before it had this many paths:
+// a report takes the host about 40 us to act on, which long kernels hide and short ones do not
+// (default scene 256^2 x 64 spp: 640 us; waiting for every report 787 us).
+#define TPT_WF_AHEAD_MIN (1u << 19)
+#define TPT_WF_MIN_LANES 8  // rays a wave takes at least when few rays are spread over the waves
 static_assert(TPT_WF_MAX_BLOCKS % TPT_WF_SEGS == 0, "grids are multiples of TPT_WF_SEGS");
 
 // Entries per queue segment for queues of at most P entries.  The shading kernel's block b
@@ -74,7 +90,8 @@ struct PathState {
   uint32_t* shl_keep;  // segmented queue of light-queue slots whose ray is traced (not self-occluded)
   uint32_t* counters;
   uint64_t* stats;  // per segment g: [g * TPT_STAT_STRIDE + k], k = 0 extension rays, 1 shadow rays, 2 paths,
-                    // 3 area-light samples, 4 of them shadowed by their own light
+                    // 3 area-light samples, 4 of them shadowed by their own light, 5 extension rays that
+                    // k_tail traced
   uint32_t seg_cap; // entries per queue segment (wf_seg_cap of the allocated path count)
   uint32_t pad;
 };
@@ -170,6 +187,14 @@ struct PassArgs {
   const int32_t* pix_map;  // image pixel of each domain pixel (null: the domain is the image)
 };
 
+// Where the kernels after a bounce's shading tell the host how many paths the next bounce has: a
+// word of pinned host memory that receives tag << 32 | paths when such a kernel starts.
+struct PathCount {
+  uint64_t* seen;  // device address (null: not told)
+  uint32_t tag;
+  int32_t queue;   // the path queue counted (0 or 1)
+};
+
 struct AccumArgs {
   uint32_t n_pixels, pixel0, k;
   double* acc;
@@ -194,13 +219,19 @@ hipError_t wf_launch_clear_radiance(const WfParams& W, uint32_t n, hipStream_t s
 // gen: the pass's paths, for the first bounce (its kernels generate the camera rays); null after
 // ev0 / ev1 (optional): events the dispatch itself records at the kernel's start and end (no
 // separate marker packets between kernels)
-hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s,
-                            hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// count: where a launch after a bounce's shading reports the next bounce's paths (all of them do, the
+// first one in time)
+hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, const PathCount& count, uint32_t max_n,
+                            hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// the rest of n paths: gen: the whole paths of a small pass; null: the paths of queue cur, whose
+// hits this bounce's extension has stored
+hipError_t wf_launch_tail(const WfParams& W, int cur, const PassArgs* gen, uint32_t n, hipStream_t s);
 hipError_t wf_launch_shade(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s);
 // cur: the queue of paths shaded this bounce; gen: the pass's paths on the first bounce (their
 // rays are generated again from their ids), null after
-hipError_t wf_launch_light_selfocc(const WfParams& W, int cur, const PassArgs* gen, uint32_t max_n, hipStream_t s);
-hipError_t wf_launch_shadow(const WfParams& W, int queue, uint32_t max_n, hipStream_t s);
+hipError_t wf_launch_light_selfocc(const WfParams& W, int cur, const PassArgs* gen, const PathCount& count,
+                                   uint32_t max_n, hipStream_t s);
+hipError_t wf_launch_shadow(const WfParams& W, int queue, const PathCount& count, uint32_t max_n, hipStream_t s);
 hipError_t wf_launch_accumulate(const WfParams& W, const AccumArgs& A, hipStream_t s);
 hipError_t wf_launch_accumulate_adaptive(const WfParams& W, const AdaptiveArgs& A, hipStream_t s);
 uint32_t wf_grid_threads(uint32_t n);
