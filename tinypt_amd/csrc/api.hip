@@ -119,7 +119,7 @@ struct tpt_scene {
   tpt_ctx* ctx = nullptr;  // null for a host-only scene (tpt_scene_build_host)
   HostScene host;
   DevBuf nodes4, tris32, tri_mat32, tri_orig, tri_inst, inst32, inst_c64, tlas_items, sph64, sph_mat;
-  DevBuf ref_nodes, ref_indices, tri_v, tri_mat, meshes, inst64;
+  DevBuf plain_nodes, plain_meshes, inst_box, ref_indices, tri_v, tri_mat, meshes, inst64;
   DevBuf mat_kind, mat_p32, mat_p64;
   DevBuf l32, cdf32, l64, cdf64;
   DevBuf env_rgb32, alias_prob, alias_idx, cell_pdf, env_rgb64, row_cdf, col_cdf;
@@ -254,7 +254,9 @@ int tpt_scene_upload(tpt_ctx* ctx, const tpt_scene_desc* desc, tpt_scene** out) 
   HIPC(upload(sc->tlas_items, H.tlas_items, s));
   HIPC(upload(sc->sph64, sph64, s));
   HIPC(upload(sc->sph_mat, H.sph_mat, s));
-  HIPC(upload(sc->ref_nodes, H.ref_nodes, s));
+  HIPC(upload(sc->plain_nodes, H.plain_nodes, s));
+  HIPC(upload(sc->plain_meshes, H.plain_meshes, s));
+  HIPC(upload(sc->inst_box, H.inst_box32, s));
   HIPC(upload(sc->ref_indices, H.ref_indices, s));
   HIPC(upload(sc->tri_v, H.tri_v, s));
   HIPC(upload(sc->tri_mat, H.tri_mat, s));
@@ -309,7 +311,7 @@ int tpt_scene_upload(tpt_ctx* ctx, const tpt_scene_desc* desc, tpt_scene** out) 
   S.n_spheres = (int32_t)H.sph_mat.size();
   // FP64 view
   SceneF64& D = sc->s64;
-  D.nodes = sc->ref_nodes.as<RefNodeDev>();
+  D.nodes = nullptr;  // the device walks plain_nodes
   D.indices = sc->ref_indices.as<int32_t>();
   D.tris = sc->tri_v.as<double>();
   D.tri_mat = sc->tri_mat.as<int32_t>();
@@ -334,7 +336,7 @@ int tpt_scene_upload(tpt_ctx* ctx, const tpt_scene_desc* desc, tpt_scene** out) 
   C.focus_dist = (float)H.cam.focus_dist;
   HIPC(hipStreamSynchronize(s));
   for (DevBuf* b : {&sc->nodes4, &sc->tris32, &sc->tri_mat32, &sc->tri_orig, &sc->tri_inst, &sc->inst32, &sc->inst_c64, &sc->tlas_items, &sc->sph64,
-                    &sc->sph_mat, &sc->ref_nodes, &sc->ref_indices, &sc->tri_v, &sc->tri_mat, &sc->meshes, &sc->inst64,
+                    &sc->sph_mat, &sc->plain_nodes, &sc->plain_meshes, &sc->inst_box, &sc->ref_indices, &sc->tri_v, &sc->tri_mat, &sc->meshes, &sc->inst64,
                     &sc->mat_kind, &sc->mat_p32, &sc->mat_p64, &sc->l32, &sc->cdf32, &sc->l64, &sc->cdf64, &sc->env_rgb32,
                     &sc->alias_prob, &sc->alias_idx, &sc->cell_pdf, &sc->env_rgb64, &sc->row_cdf, &sc->col_cdf})
     sc->device_bytes += b->bytes;
@@ -886,6 +888,9 @@ int render_plain(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* cfg, 
   HIPC(hipMemsetAsync(c->stats.p, 0, 64, s));
   Plain64Params P{};
   P.S = sc->s64;
+  P.nodes = sc->plain_nodes.as<PlainNode>();
+  P.meshes = sc->plain_meshes.as<PlainMesh>();
+  P.inst_box = sc->inst_box.as<float>();
   P.env = sc->env;
   P.lights = sc->lights;
   P.mats = sc->mats;
@@ -911,9 +916,11 @@ int render_plain(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* cfg, 
   P.welford = c->welford.as<double>();
   P.done = c->done.as<uint8_t>();
   P.stats = c->stats.as<uint64_t>();
+  plain64_shape(sc->host.max_blas_depth, &P);
   EventTimer total(s, st != nullptr, &c->ev_total);
   HIPC(total.mark());
-  const int chunk = 8;
+  // samples of a launch: about 4M paths (a launch ends with its slowest pixel), at least 8
+  const int chunk = (int)std::min<size_t>(64, std::max<size_t>(8, ((size_t)1 << 22) / npix));
   if (cfg->spp == 0) {
     P.s_begin = 0;
     P.s_end = 0;

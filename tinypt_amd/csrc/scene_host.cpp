@@ -651,6 +651,39 @@ static double mat_det(const double* m) {
 }
 static double lum(const double* c) { return 0.2126 * c[0] + 0.7152 * c[1] + 0.0722 * c[2]; }
 
+// The reference tree in the plain kernel's form (PlainNode): the inner nodes, in the reference's
+// order, each with its children's boxes.
+static PlainMesh pack_plain(const RefBvh& r, std::vector<PlainNode>& out) {
+  PlainMesh pm{};
+  pm.root = TPT_PLAIN_NONE;
+  if (r.nodes.empty()) return pm;
+  auto leaf = [](const RefNode& n) { return n.left == -1 && n.right == -1; };
+  std::vector<int32_t> rank(r.nodes.size());
+  int32_t inner = 0;
+  for (size_t i = 0; i < r.nodes.size(); i++) rank[i] = leaf(r.nodes[i]) ? TPT_PLAIN_LEAF : inner++;
+  out.resize((size_t)inner);
+  for (size_t i = 0; i < r.nodes.size(); i++) {
+    if (rank[i] < 0) continue;
+    PlainNode& o = out[(size_t)rank[i]];
+    const int32_t kids[2] = {r.nodes[i].left, r.nodes[i].right};
+    for (int k = 0; k < 2; k++) {
+      o.child[k] = TPT_PLAIN_NONE;
+      if (kids[k] < 0) continue;
+      const RefNode& c = r.nodes[(size_t)kids[k]];
+      o.child[k] = rank[(size_t)kids[k]];
+      for (int a = 0; a < 3; a++) { o.b[k][a] = c.bbox.mn[a]; o.b[k][3 + a] = c.bbox.mx[a]; }
+      o.start[k] = c.start;
+      o.count[k] = c.count;
+    }
+  }
+  const RefNode& n = r.nodes[0];
+  for (int a = 0; a < 3; a++) { pm.box[a] = n.bbox.mn[a]; pm.box[3 + a] = n.bbox.mx[a]; }
+  pm.root = rank[0];
+  pm.start = n.start;
+  pm.count = n.count;
+  return pm;
+}
+
 // ------------------------------------------------------------------ build
 bool HostScene::build(const tpt_scene_desc* d) {
   const int nm = d->n_materials, ns = d->n_spheres, nmesh = d->n_meshes, ni = d->n_instances;
@@ -743,6 +776,8 @@ bool HostScene::build(const tpt_scene_desc* d) {
   });
   std::vector<std::vector<DAabb>> bounds_of((size_t)nmesh);
   std::vector<RefBvh> sah_of((size_t)nmesh);
+  std::vector<std::vector<PlainNode>> plain_of((size_t)nmesh);
+  plain_meshes.resize((size_t)nmesh);
   {
     std::vector<std::function<void()>> tasks;
     for (int m : by_size)
@@ -755,7 +790,10 @@ bool HostScene::build(const tpt_scene_desc* d) {
     run_parallel(tasks);
     tasks.clear();
     for (int m : by_size) {
-      tasks.push_back([&, m] { blas[(size_t)m] = build_ref_bvh(bounds_of[(size_t)m], 4); });  // LEAF_SIZE (constants.rs:21)
+      tasks.push_back([&, m] {
+        blas[(size_t)m] = build_ref_bvh(bounds_of[(size_t)m], 4);  // LEAF_SIZE (constants.rs:21)
+        plain_meshes[(size_t)m] = pack_plain(blas[(size_t)m], plain_of[(size_t)m]);
+      });
       tasks.push_back([&, m] { sah_of[(size_t)m] = build_sah_bvh(bounds_of[(size_t)m], 4); });
     }
     run_parallel(tasks);
@@ -778,6 +816,10 @@ bool HostScene::build(const tpt_scene_desc* d) {
       ref_nodes.push_back(x);
     }
     for (int64_t ix : r.indices) ref_indices.push_back((int32_t)ix);
+    plain_meshes[(size_t)m].node_off = (int32_t)plain_nodes.size();
+    if (plain_nodes.empty()) plain_nodes = std::move(plain_of[(size_t)m]);
+    else plain_nodes.insert(plain_nodes.end(), plain_of[(size_t)m].begin(), plain_of[(size_t)m].end());
+    std::vector<PlainNode>().swap(plain_of[(size_t)m]);
     // the FP32 tree (own SAH build) and its reordered triangles: slot b0 + k holds triangle
     // indices[k] of that tree
     const RefBvh f = std::move(sah_of[(size_t)m]);
@@ -801,6 +843,8 @@ bool HostScene::build(const tpt_scene_desc* d) {
   inst64.resize((size_t)ni);
   inst32.resize((size_t)ni);
   inst_c64.assign(3 * (size_t)ni, 0.0);
+  inst_box32.resize(6 * (size_t)ni);
+  for (size_t k = 0; k < inst_box32.size(); k++) inst_box32[k] = k % 6 < 3 ? -INFINITY : INFINITY;
   std::vector<DAabb> item_box;
   std::vector<int32_t> item_code;
   for (int i = 0; i < ni; i++) {
@@ -831,7 +875,11 @@ bool HostScene::build(const tpt_scene_desc* d) {
     y.pad = 0;
     if (!valid || blas[(size_t)x.mesh].nodes.empty()) continue;
     const DAabb wb = instance_world_box(mesh_cut[(size_t)x.mesh], x.a, x.t);
-    for (int k = 0; k < 3; k++) inst_c64[3 * (size_t)i + k] = 0.5 * (wb.mn[k] + wb.mx[k]);
+    for (int k = 0; k < 3; k++) {
+      inst_c64[3 * (size_t)i + k] = 0.5 * (wb.mn[k] + wb.mx[k]);
+      inst_box32[6 * (size_t)i + k] = std::nextafter((float)wb.mn[k], -INFINITY);
+      inst_box32[6 * (size_t)i + 3 + k] = std::nextafter((float)wb.mx[k], INFINITY);
+    }
     item_box.push_back(wb);
     item_code.push_back(i);
   }

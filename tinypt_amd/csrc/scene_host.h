@@ -86,6 +86,9 @@ struct HostScene {
   std::vector<RefNodeDev> ref_nodes;  // all meshes' nodes, concatenated
   std::vector<int32_t> ref_indices;   // all meshes' indices (mesh-local values), concatenated
   std::vector<MeshDev> meshes;        // offsets into the concatenated arrays
+  std::vector<PlainNode> plain_nodes;  // the same trees as the plain FP64 kernel walks them
+  std::vector<PlainMesh> plain_meshes;
+  std::vector<float> inst_box32;       // 6 per instance: its world box (min, max), rounded outward
   std::vector<LightF64> lights;
   std::vector<double> light_cdf;
   double light_total = 0.0;

@@ -87,6 +87,26 @@ struct RefNodeDev {  // bvh.rs:24-35
 };
 static_assert(sizeof(RefNodeDev) == 64, "reference node is 64 B");
 
+// The reference tree as the plain FP64 kernel walks it: an inner node holds both children's boxes
+// and what they are, so that a visit is one 128 B fetch (the reference's form costs two in a row:
+// the node for its children's indices, then their boxes).
+struct alignas(16) PlainNode {
+  double b[2][6];     // child boxes: min xyz, max xyz
+  int32_t child[2];   // inner node (mesh-local), or TPT_PLAIN_LEAF / TPT_PLAIN_NONE
+  uint32_t start[2];  // leaf: its range of the mesh's indices
+  uint32_t count[2];
+  int32_t pad[2];
+};
+static_assert(sizeof(PlainNode) == 128, "plain node is 128 B");
+#define TPT_PLAIN_LEAF (-1)
+#define TPT_PLAIN_NONE (-2)
+struct PlainMesh {
+  double box[6];          // root box
+  int32_t root;           // as PlainNode::child
+  uint32_t start, count;  // of a root that is a leaf
+  int32_t node_off;       // into the plain node array
+};
+
 struct InstF64 {  // transform.rs:11-20 + world.rs:39-46
   double a[9], t[3], a_inv[9], nrm[9];
   int32_t mesh, mat_override;
