@@ -1,0 +1,48 @@
+"""Traversal kernels for small scenes (trees in LDS, rays handed to idle lanes from each wave's own
+share) against the one-ray-per-lane kernels on device memory (traversal_refill = -1): each ray's
+sequence of tests is the same, so the sums are equal bit for bit.  Scenes: a flattened tree alone
+(also one whose root is a leaf), spheres alone, both, a single triangle, nothing, the largest that
+fits the LDS and the smallest that does not.  Passes of more than 2^18 paths, since a smaller one
+goes to the kernel that walks whole paths; path counts that are no multiple of a wave."""
+import numpy as np
+import pytest
+
+import tinypt_amd as T
+from parity_scenes import PARITY_CASES, floorlight
+from tinypt_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(subdivisions):
+    return scenes.mesh_scene(64, 64, subdivisions=subdivisions, env=scenes.synthetic_env(32, 16, seed=2))
+
+
+def _without(sc, n_instances):
+    sc.world.instances = sc.world.instances[:n_instances]
+    return sc
+
+
+SCENES = {
+    "cornell": lambda: scenes.cornell_box(64, 64),
+    "spheres": lambda: scenes.default_scene(64, 64, "sky"),
+    "spheres_in_box": lambda: scenes.inverse_scene(scenes.inverse_params(3, 16), 64, 64, 16),
+    "zoo": PARITY_CASES["material_zoo"][0],
+    "root_is_a_leaf": floorlight,
+    "empty": lambda: _without(floorlight(), 0),
+    "80_triangles": lambda: _mesh(1),
+    "320_triangles": lambda: _mesh(2),
+    "1280_triangles": lambda: _mesh(3),
+}
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+@pytest.mark.parametrize("w,h,spp", [(67, 61, 131), (64, 64, 65)])
+def test_small_scene_kernels_keep_the_image(gpu_ctx, name, w, h, spp):
+    ds = T.DeviceScene(SCENES[name](), gpu_ctx)
+    kw = dict(width=w, height=h, spp=spp, max_bounces=6, rr_start=4, seed=31)
+    a, b = (T.render(ds, T.RenderConfig(traversal_refill=r, **kw)) for r in (0, -1))
+    for f in ("acc", "acc_w", "acc_sq"):
+        np.testing.assert_array_equal(getattr(a, f), getattr(b, f), err_msg=f)
+    for k in ("rays_extension", "rays_shadow", "light_samples", "light_self_occluded"):
+        assert a.stats[k] == b.stats[k], k

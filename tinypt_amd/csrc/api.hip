@@ -495,6 +495,28 @@ void refill_thresholds(const HostScene& H, int32_t requested, WfParams* W) {
   W->refill = W->refill_sh = later;
 }
 
+// The scene as the traversal kernels for small scenes hold it; bytes 0 where it does not fit, or
+// where the caller chose how rays are handed to lanes.
+SmallScene small_scene(const HostScene& H, int32_t requested_refill) {
+  SmallScene m{};
+  if (requested_refill != 0 || H.world_node0 < 0 || H.stack4 > TPT_SMALL_MAX_STACK) return m;
+  const size_t nodes = H.nodes4.size() - (size_t)H.world_node0, tris = H.tris32.size() - (size_t)H.world_tri0;
+  const size_t items = H.tlas_items.size(), sph = H.sph_mat.size();
+  if (items == 0 || nodes + tris + items + sph > TPT_SMALL_MAX_BYTES) return m;
+  const uint32_t bytes = small_scene_bytes((uint32_t)nodes, (uint32_t)tris, (uint32_t)items, (uint32_t)sph);
+  if (bytes > TPT_SMALL_MAX_BYTES) return m;
+  m.node0 = (uint32_t)H.world_node0;
+  m.n_nodes = (uint32_t)nodes;
+  m.tri0 = (uint32_t)H.world_tri0;
+  m.n_tris = (uint32_t)tris;
+  m.n_items = (uint32_t)items;
+  m.n_sph = (uint32_t)sph;
+  m.flat_root = H.flat ? H.inst32[(size_t)H.flat_inst].root : TPT_REF_EMPTY;
+  m.stack = (uint32_t)H.stack4;
+  m.bytes = bytes;
+  return m;
+}
+
 // Queue arrays hold TPT_WF_SEGS segments of wf_seg_cap(P) entries; hit and L are dense.
 int ensure_paths(PathSet* c, size_t P, int gcap) {
   if (P > c->ps_cap) {
@@ -554,6 +576,7 @@ WfParams make_wf(PathSet* c, const tpt_scene* sc, const tpt_render_config* cfg, 
   W.gstack = gcap > 0 ? c->gstack.as<int32_t>() : nullptr;
   W.gstack_cap = gcap;
   refill_thresholds(sc->host, cfg->traversal_refill, &W);
+  W.small = small_scene(sc->host, cfg->traversal_refill);
   W.width = cfg->width;
   W.height = cfg->height;
   W.max_bounces = cfg->max_bounces;

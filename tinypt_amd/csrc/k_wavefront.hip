@@ -21,7 +21,7 @@
 
 #include <algorithm>
 #include <mutex>
-#include <unordered_map>
+#include <map>
 
 namespace tpt {
 
@@ -218,9 +218,157 @@ k_extend_refill(WfParams W, int cur, PassArgs A, PathCount count) {
       continue;
     }
     if (nl == 0) break;  // the queue is taken and every lane is idle
-    if (live && !tr.step(W.S, st)) {
+    if (live && !tr.step(W.S, st, GlobalTree{W.S})) {
       W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
       live = false;
+    }
+  }
+}
+
+// ---------------------------------------------------------------- small scenes: trees in LDS
+// (measurements at k_extend_small)
+struct SmallTree {
+  static constexpr bool kWorldOnly = true;
+  const char *nodes, *tris, *sph;  // LDS, offset so that the scene's own indices address them
+  const int32_t *inst, *items;
+  int32_t root;
+  __device__ __forceinline__ uint32_t node(int32_t ref) const { return (uint32_t)ref * TPT_SMALL_NODE_BYTES; }
+  __device__ __forceinline__ float4 planes(uint32_t at) const { return *reinterpret_cast<const float4*>(nodes + (int32_t)at); }
+  __device__ __forceinline__ int4 children(uint32_t at) const {
+    return *reinterpret_cast<const int4*>(nodes + (int32_t)(at + 96u));
+  }
+  __device__ __forceinline__ const float4* tri(uint32_t slot) const {
+    return reinterpret_cast<const float4*>(tris + (int32_t)(slot * 48u));
+  }
+  __device__ __forceinline__ int32_t tri_inst(uint32_t slot) const { return inst[(int32_t)slot]; }
+  __device__ __forceinline__ int32_t item(uint32_t k) const { return items[k]; }
+  __device__ __forceinline__ const double* sphere(int32_t s) const { return reinterpret_cast<const double*>(sph + s * 32); }
+  __device__ __forceinline__ int32_t flat_root() const { return root; }
+};
+
+// Copies the scene into `mem` (every thread of the block must call it) and returns its trees and, in
+// *stack, this lane's stack behind them.
+__device__ __forceinline__ SmallTree load_small(const SceneF32& S, const SmallScene& m, float4* mem, LaneStackT<false>* stack) {
+  float4* tris = mem + m.n_nodes * (TPT_SMALL_NODE_BYTES / 16);
+  float4* sph = tris + m.n_tris * 3;
+  int32_t* inst = reinterpret_cast<int32_t*>(sph + m.n_sph * 2);
+  int32_t* items = inst + m.n_tris;
+  const float4* gn = reinterpret_cast<const float4*>(S.nodes + m.node0);
+  for (uint32_t i = threadIdx.x; i < m.n_nodes * 7; i += TPT_WF_BLOCK) mem[i] = gn[i / 7 * 8 + i % 7];
+  const float4* gt = reinterpret_cast<const float4*>(S.tris + m.tri0);
+  for (uint32_t i = threadIdx.x; i < m.n_tris * 3; i += TPT_WF_BLOCK) tris[i] = gt[i];
+  const float4* gs = reinterpret_cast<const float4*>(S.sph);
+  for (uint32_t i = threadIdx.x; i < m.n_sph * 2; i += TPT_WF_BLOCK) sph[i] = gs[i];
+  for (uint32_t i = threadIdx.x; i < m.n_tris; i += TPT_WF_BLOCK) inst[i] = S.tri_inst[m.tri0 + i];
+  for (uint32_t i = threadIdx.x; i < m.n_items; i += TPT_WF_BLOCK) items[i] = S.tlas_items[i];
+  __syncthreads();
+  *stack = LaneStackT<false>{reinterpret_cast<int32_t*>(mem + m.bytes / 16) + threadIdx.x, nullptr, TPT_WF_BLOCK,
+                             (int)m.stack};
+  return SmallTree{reinterpret_cast<const char*>(mem) - m.node0 * TPT_SMALL_NODE_BYTES,
+                   reinterpret_cast<const char*>(tris) - m.tri0 * 48u, reinterpret_cast<const char*>(sph),
+                   inst - m.tri0, items, m.flat_root};
+}
+
+// Idle lanes of a wave (with a ray ready) at which k_extend_small starts rays.
+#define TPT_SMALL_IDLE 40
+// A wave's share of n entries, handed to its lanes as they fall idle: entry groups of 64, one
+// group of every wave in turn, as a grid-stride loop takes them.  No atomics: the cursor is the
+// wave's own.
+struct WaveShare {
+  uint32_t wave, waves, taken;
+  __device__ __forceinline__ WaveShare()
+      : wave((blockIdx.x * TPT_WF_BLOCK + threadIdx.x) >> 6), waves(gridDim.x * (TPT_WF_BLOCK / 64)), taken(0) {}
+  // The next entry for this lane if it wants one; every lane of the wave must call it.
+  __device__ __forceinline__ uint32_t take(bool want) {
+    const uint64_t m = __ballot(want);
+    const uint32_t c = taken + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull));
+    taken += (uint32_t)__popcll(m);
+    return ((c >> 6) * waves + wave) * 64 + (c & 63u);
+  }
+};
+
+// k_extend for small scenes (SmallScene: at most 32 KB of trees, 20 stack entries, no instance
+// but the flattened one).  k_extend spends its issue slots on idle lanes there -- 36% of the lanes of
+// an instruction work on the Cornell box, since a wave ends with its longest ray -- and refilling
+// waves from a global cursor stall on it, on the ray loads and, vector memory answering in order,
+// then on their next node load.  Here the nodes and triangles are in LDS, whose loads are waited
+// for apart from vector memory; a lane has its next ray in registers before it needs it (loaded
+// while the wave traces); and a wave takes rays from its own share, without atomics.  A lane's new
+// ray starts once TPT_SMALL_IDLE lanes can start one.  A ray's sequence of tests is k_extend's.
+// Cornell 512^2 x 256 spp 27.1 -> 22.3 ms (started at 8 idle lanes 23.5, 16 23.4, 32 and 48 within
+// 0.3% of 40, 56 1.5% slower); its adaptive render 28.6 -> 24.2; the inverse step's 16 spheres in
+// the box and the sphere scene (bound by their short launches) unchanged.
+// GEN: the first bounce's camera rays are coherent and need no loads, so a lane takes them as
+// k_extend does.
+template <bool GEN>
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(GEN ? 5 : 6)))
+k_extend_small(WfParams W, int cur, PassArgs A, PathCount count) {
+  extern __shared__ float4 s_small[];
+  QueueMap qm;
+  uint32_t n;
+  if constexpr (GEN) {
+    n = A.n_paths;
+  } else {
+    qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
+    n = qm.n;
+  }
+  const float4* __restrict__ po = W.ps.o[cur];
+  const float4* __restrict__ pd = W.ps.d[cur];
+  LaneStackT<false> st;
+  const SmallTree tree = load_small(W.S, W.small, s_small, &st);
+  if (gtid() < TPT_WF_SEGS) {  // clear the queues the shading kernel fills next
+    W.ps.counters[TPT_CNT_IDX(cur ? TPT_CNT_Q0 : TPT_CNT_Q1, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SH, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHL, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
+  }
+  if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
+  if (!GEN) tell_count(W, count);
+  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
+  if constexpr (GEN) {
+    for (uint32_t i = gtid(); i < n; i += gridDim.x * blockDim.x) {
+      f3 o, d;
+      RngF32 rng(1);
+      gen_path(W, A, i, &rng, &o, &d);
+      HitF32 h;
+      trace_f32<false>(W.S, tree, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st);
+      W.ps.hit[i] = HitRec{__float_as_int(h.t), h.inst, h.prim};
+    }
+  } else {
+    WaveShare share;
+    TraceF32<false, SmallTree> tr;
+    f3 no = mk(0.f, 0.f, 0.f), nd = no;
+    uint32_t my = 0, nxt = share.take(true);
+    bool live = false, have = nxt < n;
+    if (have) {
+      const uint32_t slot = qm.slot(nxt);
+      no = f3of(po[slot]);
+      nd = f3of(pd[slot]);
+    }
+    for (;;) {
+      const uint64_t lm = __ballot(live), sm = __ballot(!live && have);
+      if (sm != 0 && (lm == 0 || __popcll(sm) >= TPT_SMALL_IDLE)) {  // wave-uniform
+        if (!live && have) {
+          my = nxt;
+          live = tr.init(W.S, no, nd, (float)TPT_RAY_EPSILON, 1e30f);
+          if (!live) W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
+          have = false;
+        }
+        const uint32_t t = share.take(!have);
+        if (!have && t < n) {
+          nxt = t;
+          have = true;
+          const uint32_t slot = qm.slot(t);
+          no = f3of(po[slot]);
+          nd = f3of(pd[slot]);
+        }
+        continue;
+      }
+      if (lm == 0) break;  // nothing is left to start
+      if (live && !tr.step(W.S, st, tree)) {
+        W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
+        live = false;
+      }
     }
   }
 }
@@ -762,7 +910,7 @@ k_shadow_refill(WfParams W, int queue, PathCount count) {
       continue;
     }
     if (nl == 0) break;  // the queue is taken and every lane is idle
-    if (live && !tr.step(W.S, st)) {
+    if (live && !tr.step(W.S, st, GlobalTree{W.S})) {
       if (!tr.found) add_radiance(W.ps.L, id, f3of(qc[slot]));  // unoccluded
       live = false;
     }
@@ -790,26 +938,31 @@ static inline uint32_t grid_for(uint32_t n) {
 // kernel launched with more blocks than this runs its last blocks after the first ones finish,
 // with the device partly idle (5 resident blocks per CU against 8 launched leaves a 60 %-full
 // second round); capping the grid at the resident count gives every block the same share.
-static uint32_t resident_blocks(const void* kernel) {
+static uint32_t resident_blocks(const void* kernel, uint32_t lds = 0) {
   static std::mutex mu;
-  static std::unordered_map<const void*, uint32_t> cache;  // one device model per process
+  static std::map<std::pair<const void*, uint32_t>, uint32_t> cache;  // one device model per process
   std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find(kernel);
+  auto it = cache.find({kernel, lds});
   if (it != cache.end()) return it->second;
   int dev = 0, cus = 0, per_cu = 0;
   uint32_t r = TPT_WF_MAX_BLOCKS;
   if (hipGetDevice(&dev) == hipSuccess &&
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, TPT_WF_BLOCK, 0) == hipSuccess && cus > 0 &&
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, TPT_WF_BLOCK, lds) == hipSuccess && cus > 0 &&
       per_cu > 0) {
     r = (uint32_t)cus * (uint32_t)per_cu / TPT_WF_SEGS * TPT_WF_SEGS;
     r = std::max<uint32_t>(TPT_WF_SEGS, std::min<uint32_t>(r, TPT_WF_MAX_BLOCKS));
   }
-  cache[kernel] = r;
+  cache[{kernel, lds}] = r;
   return r;
 }
 
-static inline dim3 grid_of(uint32_t n, const void* kernel) { return dim3(std::min(grid_for(n), resident_blocks(kernel))); }
+// lds: bytes of LDS that the launch adds to the kernel's own.
+static inline dim3 grid_of(uint32_t n, const void* kernel, uint32_t lds = 0) {
+  return dim3(std::min(grid_for(n), resident_blocks(kernel, lds)));
+}
+// LDS of the small-scene kernels: the scene and the lanes' stacks.
+static inline uint32_t small_lds(const WfParams& W) { return W.small.bytes + W.small.stack * TPT_WF_BLOCK * 4; }
 
 hipError_t wf_launch_clear_radiance(const WfParams& W, uint32_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_clear_radiance, dim3(grid_for(n)), dim3(TPT_WF_BLOCK), 0, s, W, n);
@@ -818,16 +971,20 @@ hipError_t wf_launch_clear_radiance(const WfParams& W, uint32_t n, hipStream_t s
 // Extension launches, timed by events that the dispatch records itself when ev0 is given.
 template <class K>
 static void launch_timed(K kernel, uint32_t max_n, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, const WfParams& W,
-                         int cur, const PassArgs& A, const PathCount& count) {
-  const dim3 grid = grid_of(max_n, (const void*)kernel);
-  if (ev0) hipExtLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, ev0, ev1, 0, W, cur, A, count);
-  else hipLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), 0, s, W, cur, A, count);
+                         int cur, const PassArgs& A, const PathCount& count, uint32_t lds = 0) {
+  const dim3 grid = grid_of(max_n, (const void*)kernel, lds);
+  if (ev0) hipExtLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), lds, s, ev0, ev1, 0, W, cur, A, count);
+  else hipLaunchKernelGGL(kernel, grid, dim3(TPT_WF_BLOCK), lds, s, W, cur, A, count);
 }
 hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, const PathCount& count, uint32_t max_n,
                             hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
   const PassArgs A = gen ? *gen : PassArgs{};
   auto launch = [&](auto kernel) { launch_timed(kernel, max_n, s, ev0, ev1, W, cur, A, count); };
-  if (gen ? W.refill_first > 0 : W.refill > 0) {
+  if (W.small.bytes > 0) {
+    const uint32_t lds = small_lds(W);
+    if (gen) launch_timed(k_extend_small<true>, max_n, s, ev0, ev1, W, cur, A, count, lds);
+    else launch_timed(k_extend_small<false>, max_n, s, ev0, ev1, W, cur, A, count, lds);
+  } else if (gen ? W.refill_first > 0 : W.refill > 0) {
     if (W.gstack) gen ? launch(k_extend_refill<true, true>) : launch(k_extend_refill<true, false>);
     else gen ? launch(k_extend_refill<false, true>) : launch(k_extend_refill<false, false>);
   } else {

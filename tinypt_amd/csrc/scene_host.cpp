@@ -888,6 +888,7 @@ bool HostScene::build(const tpt_scene_desc* d) {
   // per-instance transform, no per-instance BLAS roots.  Hits still report the original
   // instance and triangle, and ties between instances keep the reference's order (the
   // triangle's instance gives its tie key).
+  int64_t flat_tri0 = 0;
   {
     int64_t total = 0;
     for (int i = 0; i < ni; i++) {
@@ -919,7 +920,7 @@ bool HostScene::build(const tpt_scene_desc* d) {
       for (int64_t t = 0; t < total; t++) fb[(size_t)t] = triangle_bounds(&wv[9 * (size_t)t]);
       RefBvh fr = build_sah_bvh(fb, 4);
       flat_depth = fr.depth;
-      const int64_t base = (int64_t)tris32.size();
+      const int64_t base = flat_tri0 = (int64_t)tris32.size();
       tris32.resize((size_t)(base + total));
       tri_orig.resize((size_t)(base + total));
       tri_mat32.resize((size_t)(base + total));
@@ -983,6 +984,11 @@ bool HostScene::build(const tpt_scene_desc* d) {
   for (InstF32& y : inst32) {
     if (y.mesh >= 0) y.root = mesh_root2[(size_t)y.mesh];
   }
+  const bool world_only = std::all_of(tlas_items.begin(), tlas_items.end(), [&](int32_t code) {
+    return ((uint32_t)code & TPT_ITEM_SPHERE) || (flat && code == flat_inst);
+  });
+  world_node0 = world_only ? (int64_t)nodes4.size() : -1;
+  world_tri0 = flat ? flat_tri0 : (int64_t)tris32.size();
   if (flat) inst32[(size_t)flat_inst].root = collapse4(nodes2, inst32[(size_t)flat_inst].root, nodes4);
   tlas_root = collapse4(nodes2, tlas_root, nodes4);
   if (nodes4.size() > ((size_t)1 << 25)) {  // the traversal addresses nodes by 32-bit byte offsets

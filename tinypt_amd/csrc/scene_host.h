@@ -127,6 +127,10 @@ struct HostScene {
   // Root of the flattened world-space tree when the top level holds nothing else (no spheres):
   // rays then start there, without the top-level node and the instance entry.  Else
   // TPT_REF_EMPTY.
+  // First of the nodes and triangles that a ray meets when every ray stays in world space: the
+  // flattened tree's and the top level's (spheres alone: the top level's); nodes -1 if rays enter
+  // other instances.
+  int64_t world_node0 = -1, world_tri0 = 0;
   int32_t flat_only_root() const {
     return flat && sph_mat.empty() ? inst32[(size_t)flat_inst].root : TPT_REF_EMPTY;
   }

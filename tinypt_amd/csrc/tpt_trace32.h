@@ -149,6 +149,26 @@ static_assert(offsetof(Node4, hi_x) == 16 && offsetof(Node4, lo_y) == 32 && offs
                   offsetof(Node4, lo_z) == 64 && offsetof(Node4, hi_z) == 80 && offsetof(Node4, child) == 96,
               "near_off assumes the Node4 plane layout");
 
+// Where a traversal reads the scene's trees: here from device memory.  32-bit byte offsets from the
+// node array (the host keeps it under 4 GiB), so each load is the array base plus one offset
+// register.  kWorldOnly: every ray stays in world space (no instance is entered but the flattened
+// tree), so the traversal keeps one form of the ray.
+struct GlobalTree {
+  static constexpr bool kWorldOnly = false;
+  const SceneF32& S;
+  TPT_HD uint32_t node(int32_t ref) const { return (uint32_t)ref * (uint32_t)sizeof(Node4); }
+  TPT_HD float4 planes(uint32_t at) const {
+    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(S.nodes) + at);
+  }
+  TPT_HD int4 children(uint32_t at) const {
+    return *reinterpret_cast<const int4*>(reinterpret_cast<const char*>(S.nodes) + (at + 96u));
+  }
+  TPT_HD const float4* tri(uint32_t slot) const { return reinterpret_cast<const float4*>(S.tris + slot); }
+  TPT_HD int32_t tri_inst(uint32_t slot) const { return S.tri_inst[slot]; }
+  TPT_HD int32_t item(uint32_t k) const { return S.tlas_items[k]; }
+  TPT_HD const double* sphere(int32_t s) const { return S.sph + 4 * s; }
+};
+
 // One ray's traversal, resumable between steps so that a wave can swap finished rays for new
 // ones (k_extend).  ANY: stop at the first hit in range (shadow rays).
 // A step is one pass of the loop: an inner loop visits inner nodes (near child kept in `ref`, far
@@ -164,7 +184,7 @@ static_assert(offsetof(Node4, hi_x) == 16 && offsetof(Node4, lo_y) == 32 && offs
 // 32 spp 39.6 -> 36.7 ms, 4096 instances adaptive 51.7 -> 46.9, Cornell box 512^2 x 256 spp
 // 27.75 -> 27.1; two eighths 37.0, 46.6, 27.2; four 36.7, 47.4, 27.1; five 37.2, 48.5, 27.3; to
 // the last lane 42.3, 47.2, 27.7.
-template <bool ANY>
+template <bool ANY, class Tree = GlobalTree>
 struct TraceF32 {
   vec3<float> o, d, inv_w, oi_w;  // world ray
   vec3<float> co, cd, inv, oi;    // ray of the current level (object space inside an instance)
@@ -200,17 +220,24 @@ struct TraceF32 {
     tmin = rtmin;
     inv_w = mk(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
     oi_w = mk(o.x * inv_w.x, o.y * inv_w.y, o.z * inv_w.z);
-    co = o; cd = d; inv = inv_w; oi = oi_w;
     nx_w = near_off(inv_w.x, 0); ny_w = near_off(inv_w.y, 1); nz_w = near_off(inv_w.z, 2);
-    nx = nx_w; ny = ny_w; nz = nz_w;
-    lo = tmin;
-    shift = 0.f;
-    det_eps = 1e-10f;
+    to_world();
     best_t = rtmax;
     best_key = -1;
     cur_key = 0;
     sp = 0;
     return true;
+  }
+
+  // The current level is the top level or the flattened tree.
+  TPT_HD void to_world() {
+    if constexpr (!Tree::kWorldOnly) {
+      co = o; cd = d; inv = inv_w; oi = oi_w;
+      nx = nx_w; ny = ny_w; nz = nz_w;
+      lo = tmin;
+      shift = 0.f;
+      det_eps = 1e-10f;
+    }
   }
 
   TPT_HD bool at_node() const { return ref >= 0 && ref != TPT_STACK_SENTINEL; }
@@ -224,7 +251,8 @@ struct TraceF32 {
 
   // One step; false when the ray is done (hit and found hold the result).
   template <class Stack>
-  TPT_HD bool step(const SceneF32& S, const Stack& st) {
+  TPT_HD bool step(const SceneF32& S, const Stack& st, const Tree& tree) {
+    constexpr bool kWorld = Tree::kWorldOnly;
     // ---- descend inner nodes: four child boxes from one 128 B node; the nearest hit child
     // is entered, the others are pushed farthest first
     for (;;) {
@@ -235,17 +263,14 @@ struct TraceF32 {
 #else
       if (!at_node()) break;
 #endif
-      // 32-bit byte offsets from the node array (the host keeps it under 4 GiB), so each load
-      // is the array base plus one offset register
-      const char* nb = reinterpret_cast<const char*>(S.nodes);
-      const uint32_t pn = (uint32_t)ref * (uint32_t)sizeof(Node4);
-      const float4 nx4 = *reinterpret_cast<const float4*>(nb + (pn + nx));
-      const float4 fx4 = *reinterpret_cast<const float4*>(nb + (pn + (nx ^ 16u)));
-      const float4 ny4 = *reinterpret_cast<const float4*>(nb + (pn + ny));
-      const float4 fy4 = *reinterpret_cast<const float4*>(nb + (pn + (ny ^ 16u)));
-      const float4 nz4 = *reinterpret_cast<const float4*>(nb + (pn + nz));
-      const float4 fz4 = *reinterpret_cast<const float4*>(nb + (pn + (nz ^ 16u)));
-      const int4 ch = *reinterpret_cast<const int4*>(nb + (pn + 96u));
+      const uint32_t pn = tree.node(ref);
+      const uint32_t nx = kWorld ? nx_w : this->nx, ny = kWorld ? ny_w : this->ny, nz = kWorld ? nz_w : this->nz;
+      const vec3<float> inv = kWorld ? inv_w : this->inv, oi = kWorld ? oi_w : this->oi;
+      const float lo = kWorld ? tmin : this->lo;
+      const float4 nx4 = tree.planes(pn + nx), fx4 = tree.planes(pn + (nx ^ 16u));
+      const float4 ny4 = tree.planes(pn + ny), fy4 = tree.planes(pn + (ny ^ 16u));
+      const float4 nz4 = tree.planes(pn + nz), fz4 = tree.planes(pn + (nz ^ 16u));
+      const int4 ch = tree.children(pn);
       float dn[4];
       int32_t cr[4] = {ch.x, ch.y, ch.z, ch.w};
       const float bnx[4] = {nx4.x, nx4.y, nx4.z, nx4.w}, bfx[4] = {fx4.x, fx4.y, fx4.z, fx4.w};
@@ -302,17 +327,16 @@ struct TraceF32 {
     if (ref == TPT_STACK_SENTINEL) {
       // ---- leaving an instance: back to the world ray (best_t back in world units: it is the
       // best hit's distance, or the ray's tmax while nothing is hit)
-      co = o; cd = d; inv = inv_w; oi = oi_w; lo = tmin; det_eps = 1e-10f; cur_inst = -1;
-      nx = nx_w; ny = ny_w; nz = nz_w;
+      to_world();
+      cur_inst = -1;
       best_t = hit.t;
-      shift = 0.f;
     } else if (cur_inst < 0) {
       // ---- top-level leaf: one item
-      const int32_t item = S.tlas_items[(uint32_t)ref & TPT_LEAF_START_MASK];
+      const int32_t item = tree.item((uint32_t)ref & TPT_LEAF_START_MASK);
       if ((uint32_t)item & TPT_ITEM_SPHERE) {
         const int32_t s = (int32_t)((uint32_t)item & ~TPT_ITEM_SPHERE);
         double th;
-        if (sphere_hit64(S.sph + 4 * s, o, d, (double)tmin, (double)best_t, &th)) {
+        if (sphere_hit64(tree.sphere(s), o, d, (double)tmin, (double)best_t, &th)) {
           const float tf = (float)th;
           const int32_t key = TPT_KEY_SPHERE(s);
           if (tf < best_t || key >= best_key) {
@@ -322,6 +346,12 @@ struct TraceF32 {
           }
         }
       } else {
+        if constexpr (kWorld) {  // the one instance is the flattened world-space tree
+          cur_inst = item;
+          st.push(sp, TPT_STACK_SENTINEL);
+          ref = tree.flat_root();
+          return true;
+        }
         const InstF32& I = S.inst[item];
         const int32_t root = I.root;
         if (root != TPT_REF_EMPTY && item == S.flat_inst) {
@@ -374,8 +404,10 @@ struct TraceF32 {
       const uint32_t start = (uint32_t)ref & TPT_LEAF_START_MASK;
       const uint32_t cnt = (((uint32_t)ref >> 28) & 7u) + 1u;
       for (uint32_t k = 0; k < cnt; k++) {
-        const float4* tp = reinterpret_cast<const float4*>(S.tris + start + k);
+        const float4* tp = tree.tri(start + k);
         const float4 a = tp[0], b = tp[1], c = tp[2];
+        const vec3<float> co = kWorld ? o : this->co, cd = kWorld ? d : this->cd;
+        const float lo = kWorld ? tmin : this->lo, det_eps = kWorld ? 1e-10f : this->det_eps;
         // the ray in the triangle's frame (TriF32): the plane at w = 0, the triangle where
         // u, v >= 0 and u + v <= 1 -- the hits of Triangle::hit (geometry.rs:236-273) up to
         // rounding; comparisons written so that NaN (degenerate triangles, rays in the
@@ -391,14 +423,14 @@ struct TraceF32 {
         const float v = fmaf(th, b.x * cd.x + b.y * cd.y + b.z * cd.z, b.x * tv.x + b.y * tv.y + b.z * tv.z);
         if (!(v >= 0.f && u + v <= 1.f)) continue;
         int32_t key = cur_key, hinst = cur_inst;
-        if (cur_inst == S.flat_inst) {  // world-space triangle: its own instance decides ties
-          const int32_t i0 = S.tri_inst[start + k] & (int32_t)~TPT_TRI_FLIP;
+        if (kWorld || cur_inst == S.flat_inst) {  // world-space triangle: its own instance decides ties
+          const int32_t i0 = tree.tri_inst(start + k) & (int32_t)~TPT_TRI_FLIP;
           key = TPT_KEY_INST(i0);
           hinst = (int32_t)((uint32_t)i0 | TPT_HIT_FLAT);
         }
         if (th < best_t || key >= best_key) {
           best_t = th; best_key = key; found = true;
-          hit.t = th + shift; hit.inst = hinst; hit.prim = (int32_t)(start + k);
+          hit.t = kWorld ? th : th + shift; hit.inst = hinst; hit.prim = (int32_t)(start + k);
           if (ANY) return false;
         }
       }
@@ -408,16 +440,21 @@ struct TraceF32 {
 };
 
 // Returns true on a hit.  ANY: stop at the first hit in range (shadow rays).
-template <bool ANY, class Stack>
-TPT_HD bool trace_f32(const SceneF32& S, vec3<float> o, vec3<float> d, float tmin, float tmax, HitF32* hit,
-                      const Stack& st) {
-  TraceF32<ANY> tr;
+template <bool ANY, class Tree, class Stack>
+TPT_HD bool trace_f32(const SceneF32& S, const Tree& tree, vec3<float> o, vec3<float> d, float tmin, float tmax,
+                      HitF32* hit, const Stack& st) {
+  TraceF32<ANY, Tree> tr;
   if (tr.init(S, o, d, tmin, tmax)) {
-    while (tr.step(S, st)) {
+    while (tr.step(S, st, tree)) {
     }
   }
   *hit = tr.hit;
   return tr.found;
+}
+template <bool ANY, class Stack>
+TPT_HD bool trace_f32(const SceneF32& S, vec3<float> o, vec3<float> d, float tmin, float tmax, HitF32* hit,
+                      const Stack& st) {
+  return trace_f32<ANY>(S, GlobalTree{S}, o, d, tmin, tmax, hit, st);
 }
 
 }  // namespace tpt
