@@ -473,26 +473,16 @@ int needed_gstack(const HostScene& H) {
   return need > TPT_WF_STACK ? need - TPT_WF_STACK : 0;
 }
 
-// Lanes below which a wave of the persistent traversal kernels takes new rays (0: one ray per
-// lane, the plain kernels), for the first bounce's extension, the later extensions and the
-// shadow rays.  Refilling pays where the rays of a wave need very different amounts of work and
-// costs a global cursor atomic per refill.  Measured on MI355X (FP32 form, images unchanged): a
-// two-level scene of 4096 instances (top-level depth 16, 3.4M BLAS nodes) at 48 -- extension
-// -17%, shadow rays -9%, adaptive render 26.3 -> 19.0 s (its adaptive passes' camera rays, of
-// scattered active pixels, gain too); a single tree of 1.31M triangles at 16 -- later bounces
-// -5%, shadow rays -17%, but its first bounce, coherent camera rays, 75% slower, so that one
-// keeps one ray per lane; the 36-triangle Cornell box at 16 -- extension 2.1x slower (its rays
-// finish within a few steps, so waves refill almost every step).
-void refill_thresholds(const HostScene& H, int32_t requested, WfParams* W) {
-  int32_t first = 0, later = 0;
-  if (requested > 0) {
-    first = later = std::min(requested, 63);
-  } else if (requested == 0) {
-    if (!H.flat && H.inst32.size() >= 64) first = later = 48;
-    else if (H.stack4 > TPT_WF_STACK) later = 16;
-  }
-  W->refill_first = first;
-  W->refill = W->refill_sh = later;
+// Lanes below which a wave of the persistent traversal kernels starts new rays, for the extension
+// rays after the first bounce and the shadow rays (0: one ray per lane, the plain kernels).  They pay
+// where the rays of a wave need very different amounts of work.  Measured on MI355X (images
+// unchanged): 1.31M-triangle mesh 1080p x 32 spp 33.3 ms at 48 lanes (24: 33.7, 16: 35.1), 4096
+// instances adaptive 38.9 at 48 (32: 40.2); 512^2 x 32 spp with these kernels against one ray per lane:
+// an 82k-triangle mesh 6.76 ms against 7.14; trees within the LDS stack: 5k triangles 4.70 against
+// 4.57, 1280 triangles 4.20 against 3.92.
+int32_t refill_lanes(const HostScene& H, int32_t requested) {
+  if (requested != 0) return requested < 0 ? 0 : std::min(requested, 63);
+  return (!H.flat && H.inst32.size() >= 64) || H.stack4 > TPT_WF_STACK ? 48 : 0;
 }
 
 // The scene as the traversal kernels for small scenes hold it; bytes 0 where it does not fit, or
@@ -575,7 +565,7 @@ WfParams make_wf(PathSet* c, const tpt_scene* sc, const tpt_render_config* cfg, 
   ps.seg_cap = wf_seg_cap((uint32_t)c->ps_cap);
   W.gstack = gcap > 0 ? c->gstack.as<int32_t>() : nullptr;
   W.gstack_cap = gcap;
-  refill_thresholds(sc->host, cfg->traversal_refill, &W);
+  W.refill = refill_lanes(sc->host, cfg->traversal_refill);
   W.small = small_scene(sc->host, cfg->traversal_refill);
   W.width = cfg->width;
   W.height = cfg->height;

@@ -101,6 +101,20 @@ __device__ __forceinline__ void tell_count(const WfParams& W, const PathCount& c
   __hip_atomic_store(c.seen, (uint64_t)c.tag << 32 | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Every extension kernel: clears the queues that the shading kernel fills next, reports the paths,
+// counts the n rays.
+template <bool GEN>
+__device__ __forceinline__ void begin_extension(const WfParams& W, int cur, uint32_t n, const PathCount& count) {
+  if (gtid() < TPT_WF_SEGS) {
+    W.ps.counters[TPT_CNT_IDX(cur ? TPT_CNT_Q0 : TPT_CNT_Q1, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SH, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHL, gtid())] = 0;
+    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
+  }
+  if (!GEN) tell_count(W, count);
+  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
+}
+
 // OVF: the scene's stack bound exceeds the LDS part, so the traversal stack may overflow to the
 // per-thread global area (W.gstack); otherwise that path is compiled out.  GEN: the first
 // bounce, whose paths are the pass's camera rays, generated here (path i at position i).  Six
@@ -122,15 +136,7 @@ k_extend(WfParams W, int cur, PassArgs A, PathCount count) {
   const float4* __restrict__ pd = W.ps.d[cur];
   LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
                      TPT_WF_STACK};
-  if (gtid() < TPT_WF_SEGS) {  // clear the queues the shading kernel fills next
-    W.ps.counters[TPT_CNT_IDX(cur ? TPT_CNT_Q0 : TPT_CNT_Q1, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SH, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHL, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
-  }
-  if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
-  if (!GEN) tell_count(W, count);
-  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
+  begin_extension<GEN>(W, cur, n, count);
   for (uint32_t i = gtid(); i < n; i += gridDim.x * blockDim.x) {
     f3 o, d;
     if constexpr (GEN) {
@@ -144,84 +150,6 @@ k_extend(WfParams W, int cur, PassArgs A, PathCount count) {
     HitF32 h;
     trace_f32<false>(W.S, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st);
     W.ps.hit[i] = HitRec{__float_as_int(h.t), h.inst, h.prim};
-  }
-}
-
-// Persistent form of k_extend for deep trees, where the rays of one wave need very different
-// numbers of traversal steps: a wave keeps its lanes' traversals resumable (TraceF32 step by
-// step) and, once fewer than T lanes are still tracing (W.refill, or W.refill_first on the first
-// bounce), hands its idle lanes the next rays of the queue (one atomic per refill on a global
-// cursor; dynamic ray fetch, Aila and Laine 2009).  The hits are those of k_extend: each ray's traversal is the same sequence of steps.
-// The cursor (TPT_CNT_FETCH) is zero at launch: the render clears it, and every k_shade and
-// k_accumulate launch clears it for the next extension launch.  Every wave exits once the cursor has passed the
-// queue's end and its lanes are idle.  With the overflow path the resumable state needs more
-// registers: five waves per SIMD (96 VGPRs) for the later bounces and four (117) for the first
-// keep it out of scratch, where six and five spilled 44 and 64 bytes per lane that the loop
-// reloaded at every step (measured: the 1.31M-triangle mesh 4% and the 4096 instances 11%
-// faster).
-template <bool OVF, bool GEN>
-__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(GEN && OVF ? 4 : GEN || OVF ? 5 : 6)))
-k_extend_refill(WfParams W, int cur, PassArgs A, PathCount count) {
-  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
-  QueueMap qm;
-  uint32_t n;
-  if constexpr (GEN) {
-    n = A.n_paths;
-  } else {
-    qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
-    n = qm.n;
-  }
-  const float4* __restrict__ po = W.ps.o[cur];
-  const float4* __restrict__ pd = W.ps.d[cur];
-  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
-                     TPT_WF_STACK};
-  if (gtid() < TPT_WF_SEGS) {  // clear the queues the shading kernel fills next
-    W.ps.counters[TPT_CNT_IDX(cur ? TPT_CNT_Q0 : TPT_CNT_Q1, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SH, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHL, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
-  }
-  if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
-  if (!GEN) tell_count(W, count);
-  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
-  uint32_t* cursor = W.ps.counters + TPT_CNT_FETCH;
-  const uint32_t lane = __lane_id();
-  TraceF32<false> tr;
-  bool live = false, exhausted = false;
-  uint32_t my = 0;
-  // nl < threshold <= 64: every refill moves the cursor
-  const int threshold = min(GEN ? W.refill_first : W.refill, 64);
-  for (;;) {
-    const uint64_t mask = __ballot(live);
-    const int nl = __popcll(mask);
-    if (!exhausted && nl < threshold) {  // wave-uniform: refill the idle lanes
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(cursor, (uint32_t)(64 - nl));
-      base = (uint32_t)__shfl((int)base, 0);
-      if (base >= n) exhausted = true;
-      if (!live) {
-        my = base + (uint32_t)__popcll(~mask & ((1ull << lane) - 1ull));
-        if (my < n) {
-          f3 o, d;
-          if constexpr (GEN) {
-            RngF32 rng(1);
-            gen_path(W, A, my, &rng, &o, &d);
-          } else {
-            const uint32_t slot = qm.slot(my);
-            o = f3of(po[slot]);
-            d = f3of(pd[slot]);
-          }
-          live = tr.init(W.S, o, d, (float)TPT_RAY_EPSILON, 1e30f);
-          if (!live) W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
-        }
-      }
-      continue;
-    }
-    if (nl == 0) break;  // the queue is taken and every lane is idle
-    if (live && !tr.step(W.S, st, GlobalTree{W.S})) {
-      W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
-      live = false;
-    }
   }
 }
 
@@ -269,9 +197,9 @@ __device__ __forceinline__ SmallTree load_small(const SceneF32& S, const SmallSc
                    inst - m.tri0, items, m.flat_root};
 }
 
-// Idle lanes of a wave (with a ray ready) at which k_extend_small and k_shadow_small start rays.
-#define TPT_SMALL_IDLE 40
-#define TPT_SMALL_IDLE_SH 48
+// A wave of k_extend_small / k_shadow_small starts rays once fewer lanes than this are tracing.
+#define TPT_SMALL_LANES 25
+#define TPT_SMALL_LANES_SH 17
 // A wave's share of n entries, handed to its lanes as they fall idle: entry groups of 64, one
 // group of every wave in turn, as a grid-stride loop takes them.  No atomics: the cursor is the
 // wave's own.
@@ -287,6 +215,51 @@ struct WaveShare {
     return ((c >> 6) * waves + wave) * 64 + (c & 63u);
   }
 };
+
+// The rays of a wave's share of queue cur, each lane's traversal resumable (TraceF32 step by step):
+// once fewer than `lanes` lanes are tracing, the idle ones start their next rays, which they have
+// held in registers since the last start, so that the wave does not wait for the load.
+template <class Tree, class Stack>
+__device__ __forceinline__ void extend_share(const WfParams& W, int cur, const Tree& tree, const Stack& st, int lanes) {
+  QueueMap qm;
+  qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
+  const float4* __restrict__ po = W.ps.o[cur];
+  const float4* __restrict__ pd = W.ps.d[cur];
+  WaveShare share;
+  TraceF32<false, Tree> tr;
+  f3 no = mk(0.f, 0.f, 0.f), nd = no;
+  uint32_t my = 0, nxt = 0;
+  bool live = false, have = false;
+  auto fetch = [&]() {  // every lane of the wave
+    const uint32_t t = share.take(!have);
+    if (have || t >= qm.n) return;
+    nxt = t;
+    have = true;
+    const uint32_t slot = qm.slot(t);
+    no = f3of(po[slot]);
+    nd = f3of(pd[slot]);
+  };
+  fetch();
+  for (;;) {
+    const int nl = __popcll(__ballot(live));
+    const bool some = __ballot(!live && have) != 0;
+    if (some && nl < lanes) {  // wave-uniform
+      if (!live && have) {
+        my = nxt;
+        have = false;
+        live = tr.init(W.S, no, nd, (float)TPT_RAY_EPSILON, 1e30f);
+        if (!live) W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
+      }
+      fetch();
+      continue;
+    }
+    if (nl == 0) break;  // the share is taken and every lane is idle
+    if (live && !tr.step(W.S, st, tree)) {
+      W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
+      live = false;
+    }
+  }
+}
 
 // k_extend for small scenes (SmallScene: at most 32 KB of trees, 20 stack entries, no instance
 // but the flattened one).  k_extend spends its issue slots on idle lanes there -- 36% of the lanes of
@@ -313,19 +286,9 @@ k_extend_small(WfParams W, int cur, PassArgs A, PathCount count) {
     qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
     n = qm.n;
   }
-  const float4* __restrict__ po = W.ps.o[cur];
-  const float4* __restrict__ pd = W.ps.d[cur];
   LaneStackT<false> st;
   const SmallTree tree = load_small(W.S, W.small, s_small, &st);
-  if (gtid() < TPT_WF_SEGS) {  // clear the queues the shading kernel fills next
-    W.ps.counters[TPT_CNT_IDX(cur ? TPT_CNT_Q0 : TPT_CNT_Q1, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SH, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHL, gtid())] = 0;
-    W.ps.counters[TPT_CNT_IDX(TPT_CNT_SHK, gtid())] = 0;
-  }
-  if (gtid() < 2) W.ps.counters[TPT_CNT_FETCH_SH(gtid())] = 0;  // cursors of this bounce's shadow kernels
-  if (!GEN) tell_count(W, count);
-  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[0], (unsigned long long)n);
+  begin_extension<GEN>(W, cur, n, count);
   if constexpr (GEN) {
     for (uint32_t i = gtid(); i < n; i += gridDim.x * blockDim.x) {
       f3 o, d;
@@ -336,42 +299,30 @@ k_extend_small(WfParams W, int cur, PassArgs A, PathCount count) {
       W.ps.hit[i] = HitRec{__float_as_int(h.t), h.inst, h.prim};
     }
   } else {
-    WaveShare share;
-    TraceF32<false, SmallTree> tr;
-    f3 no = mk(0.f, 0.f, 0.f), nd = no;
-    uint32_t my = 0, nxt = share.take(true);
-    bool live = false, have = nxt < n;
-    if (have) {
-      const uint32_t slot = qm.slot(nxt);
-      no = f3of(po[slot]);
-      nd = f3of(pd[slot]);
-    }
-    for (;;) {
-      const uint64_t lm = __ballot(live), sm = __ballot(!live && have);
-      if (sm != 0 && (lm == 0 || __popcll(sm) >= TPT_SMALL_IDLE)) {  // wave-uniform
-        if (!live && have) {
-          my = nxt;
-          live = tr.init(W.S, no, nd, (float)TPT_RAY_EPSILON, 1e30f);
-          if (!live) W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
-          have = false;
-        }
-        const uint32_t t = share.take(!have);
-        if (!have && t < n) {
-          nxt = t;
-          have = true;
-          const uint32_t slot = qm.slot(t);
-          no = f3of(po[slot]);
-          nd = f3of(pd[slot]);
-        }
-        continue;
-      }
-      if (lm == 0) break;  // nothing is left to start
-      if (live && !tr.step(W.S, st, tree)) {
-        W.ps.hit[my] = HitRec{__float_as_int(tr.hit.t), tr.hit.inst, tr.hit.prim};
-        live = false;
-      }
-    }
+    extend_share(W, cur, tree, st, TPT_SMALL_LANES);
   }
+}
+
+// Persistent form of k_extend for the later bounces of deep trees, where the rays of one wave need
+// very different numbers of traversal steps: lanes that fall idle go on with the next rays of their
+// wave's share once fewer than W.refill lanes are tracing (persistent threads, Aila and Laine 2009).
+// The hits are those of k_extend: each ray's traversal is the same sequence of steps.  Against taking
+// rays from one global cursor -- an atomic's and a ray load's way to memory, one after the other, for
+// the whole wave at every start -- on MI355X: 1.31M-triangle mesh 1080p x 32 spp 36.7 -> 33.3 ms, 4096
+// instances adaptive 46.7 -> 38.9, 20k-triangle mesh 333x217 x 50 spp 3.45 -> 2.74.  The ray held
+// ahead needs the registers of four waves per SIMD with the overflow path (five, spilling 44 B a
+// lane: the instances 41.5).  The first bounce keeps one ray per lane: its camera rays are coherent
+// (as shares: the mesh 35.8 ms, the instances 39.1).
+template <bool OVF>
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(OVF ? 4 : 5)))
+k_extend_refill(WfParams W, int cur, PassArgs, PathCount count) {
+  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
+  QueueMap qm;
+  qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
+  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
+                     TPT_WF_STACK};
+  begin_extension<false>(W, cur, qm.n, count);
+  extend_share(W, cur, GlobalTree{W.S}, st, W.refill);
 }
 
 __device__ __forceinline__ void add_radiance(float4* L, int32_t id, f3 c) {
@@ -525,7 +476,6 @@ k_shade(WfParams W, int cur, PassArgs A) {
   }
   const int nxt = cur ^ 1;
   const uint32_t stride = gridDim.x * blockDim.x;
-  if (gtid() == 0) W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next extension launch (k_extend_refill)
   for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
     const uint32_t i = base + threadIdx.x;
     // path state (valid when i < n)
@@ -681,26 +631,20 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_
               (unsigned long long)tot);
 }
 
-// k_shadow for small scenes, see k_extend_small.  A lane's next ray is loaded one start ahead (the
-// light queue's list of surviving slots two ahead), and the radiance of the rays that were found
-// unoccluded is added when the next rays start, so that the wave waits for that read once for
-// many rays.  Cornell 512^2 x 256 spp 22.3 -> 21.5 ms; the look-ahead needs the registers of four
-// waves per SIMD (at five, with spills, 22.0; at six 23.0); started at 8 idle lanes 22.5, 32 and
-// 56 within 0.3% of 48.
-__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-k_shadow_small(WfParams W, int queue, PathCount count) {
-  extern __shared__ float4 s_small[];
-  tell_count(W, count);
+// The shadow rays of a wave's share, as extend_share: a lane's next ray is loaded one start ahead
+// (the light queue's list of surviving slots two ahead), and the radiance of the rays that were
+// found unoccluded is added when the next rays start, so that the wave waits for that read once for
+// many rays.
+template <class Tree, class Stack>
+__device__ __forceinline__ void shadow_share(const WfParams& W, int queue, const Tree& tree, const Stack& st, int lanes) {
   QueueMap qm;
   qm.load(W.ps.counters, queue ? TPT_CNT_SHK : TPT_CNT_SH, W.ps.seg_cap);
   const uint32_t n = qm.n;
   const float4* __restrict__ qo = queue ? W.ps.sh_l : W.ps.sh_o[0];
   const float4* __restrict__ qd = W.ps.sh_d[queue];
   const float4* __restrict__ qc = W.ps.sh_c[queue];
-  LaneStackT<false> st;
-  const SmallTree tree = load_small(W.S, W.small, s_small, &st);
   WaveShare share;
-  TraceF32<true, SmallTree> tr;
+  TraceF32<true, Tree> tr;
   uint32_t traced = 0;
   bool live = false, lit = false;  // lit: the lane's last ray was unoccluded, its radiance is still to be added
   uint32_t slot = 0;
@@ -733,8 +677,9 @@ k_shadow_small(WfParams W, int queue, PathCount count) {
   fetch_ray(true);
   fetch_slot(true);
   for (;;) {
-    const uint64_t lm = __ballot(live), sm = __ballot(!live && have);
-    if (lm == 0 || (sm != 0 && __popcll(sm) >= TPT_SMALL_IDLE_SH)) {  // wave-uniform
+    const int nl = __popcll(__ballot(live));
+    const bool some = __ballot(!live && have) != 0;
+    if (nl == 0 || (some && nl < lanes)) {  // wave-uniform
       const bool start = !live && have;
       const bool add = !live && lit;
       float4 l, c;
@@ -764,7 +709,7 @@ k_shadow_small(WfParams W, int queue, PathCount count) {
       const bool want = !have;
       fetch_ray(want);
       fetch_slot(want);
-      if (sm == 0) break;  // nothing was started
+      if (!some) break;  // nothing was started: the share is taken
       continue;
     }
     if (live && !tr.step(W.S, st, tree)) {
@@ -777,6 +722,30 @@ k_shadow_small(WfParams W, int queue, PathCount count) {
   if (__lane_id() == 0 && tot)
     atomicAdd((unsigned long long*)&W.ps.stats[(blockIdx.x & (TPT_WF_SEGS - 1)) * TPT_STAT_STRIDE + 1],
               (unsigned long long)tot);
+}
+
+// k_shadow for small scenes, see k_extend_small.
+// Cornell 512^2 x 256 spp 22.3 -> 21.5 ms; the look-ahead needs the registers of four
+// waves per SIMD (at five, with spills, 22.0; at six 23.0); started at 8 idle lanes 22.5, 32 and
+// 56 within 0.3% of 48.
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+k_shadow_small(WfParams W, int queue, PathCount count) {
+  extern __shared__ float4 s_small[];
+  tell_count(W, count);
+  LaneStackT<false> st;
+  const SmallTree tree = load_small(W.S, W.small, s_small, &st);
+  shadow_share(W, queue, tree, st, TPT_SMALL_LANES_SH);
+}
+
+// k_shadow for deep trees, see k_extend_refill.
+template <bool OVF>
+__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+k_shadow_refill(WfParams W, int queue, PathCount count) {
+  tell_count(W, count);
+  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
+  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
+                     TPT_WF_STACK};
+  shadow_share(W, queue, GlobalTree{W.S}, st, W.refill);
 }
 
 // The rest of a few paths in one launch: each lane walks its path to the end -- extension, shading,
@@ -896,7 +865,6 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate(WfParams W, AccumAr
     if (A.acc_sq) { A.acc_sq[3 * g_pix] += r2; A.acc_sq[3 * g_pix + 1] += g2; A.acc_sq[3 * g_pix + 2] += b2; }
   }
   if (gtid() == 0) {
-    W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next pass
     atomicAdd((unsigned long long*)&W.ps.stats[2], (unsigned long long)A.n_pixels * A.k);
   }
 }
@@ -908,7 +876,6 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate_adaptive(WfParams W
   __shared__ uint32_t s_slot[8];
   const uint32_t stride = gridDim.x * blockDim.x;
   uint32_t kept = 0;  // samples this thread added to its pixels (the paths the render counts)
-  if (gtid() == 0) W.ps.counters[TPT_CNT_FETCH] = 0;  // for the next pass
   for (uint32_t base = blockIdx.x * blockDim.x; base < A.n_active; base += stride) {
     uint32_t j = base + threadIdx.x;
     bool keep = false;
@@ -956,69 +923,6 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate_adaptive(WfParams W
   if (__lane_id() == 0 && kept)
     atomicAdd((unsigned long long*)&W.ps.stats[(blockIdx.x & (TPT_WF_SEGS - 1)) * TPT_STAT_STRIDE + 2],
               (unsigned long long)kept);
-}
-
-// Persistent form of k_shadow for deep trees (see k_extend_refill): lanes whose shadow ray is
-// done take the queue's next rays once fewer than W.refill_sh lanes are still tracing.  The
-// cursor TPT_CNT_FETCH_SH(queue) is cleared by the extension kernel of the same bounce.
-template <bool OVF>
-__global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
-k_shadow_refill(WfParams W, int queue, PathCount count) {
-  tell_count(W, count);
-  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
-  QueueMap qm;
-  qm.load(W.ps.counters, queue ? TPT_CNT_SHK : TPT_CNT_SH, W.ps.seg_cap);
-  const uint32_t n = qm.n;
-  const float4* __restrict__ qo = queue ? W.ps.sh_l : W.ps.sh_o[0];
-  const float4* __restrict__ qd = W.ps.sh_d[queue];
-  const float4* __restrict__ qc = W.ps.sh_c[queue];
-  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
-                     TPT_WF_STACK};
-  uint32_t* cursor = W.ps.counters + TPT_CNT_FETCH_SH(queue);
-  const uint32_t lane = __lane_id();
-  TraceF32<true> tr;
-  bool live = false, exhausted = false;
-  uint32_t slot = 0, traced = 0;
-  int32_t id = 0;
-  const int threshold = min(W.refill_sh, 64);  // nl < threshold <= 64: every refill moves the cursor
-  for (;;) {
-    const uint64_t mask = __ballot(live);
-    const int nl = __popcll(mask);
-    if (!exhausted && nl < threshold) {  // wave-uniform: refill the idle lanes
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(cursor, (uint32_t)(64 - nl));
-      base = (uint32_t)__shfl((int)base, 0);
-      if (base >= n) exhausted = true;
-      if (!live) {
-        const uint32_t j = base + (uint32_t)__popcll(~mask & ((1ull << lane) - 1ull));
-        if (j < n) {
-          slot = queue ? W.ps.shl_keep[qm.slot(j)] : qm.slot(j);
-          const float4 o4 = qo[slot], d4 = qd[slot];
-          f3 o = f3of(o4);
-          float tmax = o4.w;
-          if (queue) {  // light queue: o4 is the shading point, sh_c's w the distance to the light sample
-            o = o + (float)TPT_RAY_EPSILON * f3of(d4);
-            tmax = light_shadow_tmax32(qc[slot].w);
-          }
-          id = __float_as_int(d4.w);
-          traced++;
-          live = tr.init(W.S, o, f3of(d4), (float)TPT_RAY_EPSILON, tmax);
-          if (!live && !tr.found) add_radiance(W.ps.L, id, f3of(qc[slot]));
-        }
-      }
-      continue;
-    }
-    if (nl == 0) break;  // the queue is taken and every lane is idle
-    if (live && !tr.step(W.S, st, GlobalTree{W.S})) {
-      if (!tr.found) add_radiance(W.ps.L, id, f3of(qc[slot]));  // unoccluded
-      live = false;
-    }
-  }
-  uint32_t tot = traced;
-  for (int off = 32; off > 0; off >>= 1) tot += (uint32_t)__shfl_down((int)tot, off);
-  if (__lane_id() == 0 && tot)
-    atomicAdd((unsigned long long*)&W.ps.stats[(blockIdx.x & (TPT_WF_SEGS - 1)) * TPT_STAT_STRIDE + 1],
-              (unsigned long long)tot);
 }
 
 // ---------------------------------------------------------------- host-side launchers
@@ -1083,9 +987,8 @@ hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, con
     const uint32_t lds = small_lds(W);
     if (gen) launch_timed(k_extend_small<true>, max_n, s, ev0, ev1, W, cur, A, count, lds);
     else launch_timed(k_extend_small<false>, max_n, s, ev0, ev1, W, cur, A, count, lds);
-  } else if (gen ? W.refill_first > 0 : W.refill > 0) {
-    if (W.gstack) gen ? launch(k_extend_refill<true, true>) : launch(k_extend_refill<true, false>);
-    else gen ? launch(k_extend_refill<false, true>) : launch(k_extend_refill<false, false>);
+  } else if (!gen && W.refill > 0) {
+    W.gstack ? launch(k_extend_refill<true>) : launch(k_extend_refill<false>);
   } else {
     if (W.gstack) gen ? launch(k_extend<true, true>) : launch(k_extend<true, false>);
     else gen ? launch(k_extend<false, true>) : launch(k_extend<false, false>);
@@ -1142,7 +1045,7 @@ hipError_t wf_launch_shadow(const WfParams& W, int queue, const PathCount& count
     launch(k_shadow_small, small_lds(W));
     return hipGetLastError();
   }
-  if (W.refill_sh > 0) W.gstack ? launch(k_shadow_refill<true>) : launch(k_shadow_refill<false>);
+  if (W.refill > 0) W.gstack ? launch(k_shadow_refill<true>) : launch(k_shadow_refill<false>);
   else W.gstack ? launch(k_shadow<true>) : launch(k_shadow<false>);
   return hipGetLastError();
 }

@@ -186,9 +186,10 @@ struct GlobalTree {
 // the last lane 42.3, 47.2, 27.7.
 template <bool ANY, class Tree = GlobalTree>
 struct TraceF32 {
-  vec3<float> o, d, inv_w, oi_w;  // world ray
-  vec3<float> co, cd, inv, oi;    // ray of the current level (object space inside an instance)
-  uint32_t nx_w, ny_w, nz_w, nx, ny, nz;
+  vec3<float> o, d;        // world ray
+  vec3<float> co, cd;      // ray of the current level (object space inside an instance; unused if kWorldOnly)
+  vec3<float> inv, oi;     // of the current level: 1 / d, o / d
+  uint32_t nx, ny, nz;     // ... and its near planes (near_off)
   float tmin;
   float shift;    // world t of the current level's origin (0 at the top level)
   float lo;       // lower t bound at the current level
@@ -218,9 +219,6 @@ struct TraceF32 {
     o = ro;
     d = rd;
     tmin = rtmin;
-    inv_w = mk(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-    oi_w = mk(o.x * inv_w.x, o.y * inv_w.y, o.z * inv_w.z);
-    nx_w = near_off(inv_w.x, 0); ny_w = near_off(inv_w.y, 1); nz_w = near_off(inv_w.z, 2);
     to_world();
     best_t = rtmax;
     best_key = -1;
@@ -229,11 +227,16 @@ struct TraceF32 {
     return true;
   }
 
-  // The current level is the top level or the flattened tree.
+  // The current level is the top level or the flattened tree.  Computed again on the way out of an
+  // instance rather than kept: nine registers that a deep tree's kernel has better use for.
   TPT_HD void to_world() {
+    vec3<float> o = this->o, d = this->d;
+    opaque(o.x); opaque(o.y); opaque(o.z); opaque(d.x); opaque(d.y); opaque(d.z);
+    inv = mk(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
+    oi = mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+    nx = near_off(inv.x, 0); ny = near_off(inv.y, 1); nz = near_off(inv.z, 2);
     if constexpr (!Tree::kWorldOnly) {
-      co = o; cd = d; inv = inv_w; oi = oi_w;
-      nx = nx_w; ny = ny_w; nz = nz_w;
+      co = o; cd = d;
       lo = tmin;
       shift = 0.f;
       det_eps = 1e-10f;
@@ -264,8 +267,6 @@ struct TraceF32 {
       if (!at_node()) break;
 #endif
       const uint32_t pn = tree.node(ref);
-      const uint32_t nx = kWorld ? nx_w : this->nx, ny = kWorld ? ny_w : this->ny, nz = kWorld ? nz_w : this->nz;
-      const vec3<float> inv = kWorld ? inv_w : this->inv, oi = kWorld ? oi_w : this->oi;
       const float lo = kWorld ? tmin : this->lo;
       const float4 nx4 = tree.planes(pn + nx), fx4 = tree.planes(pn + (nx ^ 16u));
       const float4 ny4 = tree.planes(pn + ny), fy4 = tree.planes(pn + (ny ^ 16u));
@@ -327,7 +328,7 @@ struct TraceF32 {
     if (ref == TPT_STACK_SENTINEL) {
       // ---- leaving an instance: back to the world ray (best_t back in world units: it is the
       // best hit's distance, or the ray's tmax while nothing is hit)
-      to_world();
+      if constexpr (!kWorld) to_world();
       cur_inst = -1;
       best_t = hit.t;
     } else if (cur_inst < 0) {
@@ -362,8 +363,6 @@ struct TraceF32 {
           return true;
         }
         if (root != TPT_REF_EMPTY) {
-          const float4* w = reinterpret_cast<const float4*>(I.w2o);
-          const float4 r0 = w[0], r1 = w[1], r2 = w[2];
           // re-base the origin in FP64 to o + s d, the ray's point nearest the instance's
           // centre c (s is an FP32 number, so that the shift of t is exactly s; any s near
           // the nearest point serves, so |d|^2 is divided by with an approximate reciprocal)
@@ -380,11 +379,12 @@ struct TraceF32 {
             const double s = shift;
             const double px = ox + s * dx - J.t[0], py = oy + s * dy - J.t[1], pz = oz + s * dz - J.t[2];
             const double* m = J.a_inv;
+            cd = mk(fmaf((float)m[0], d.x, fmaf((float)m[1], d.y, (float)m[2] * d.z)),
+                    fmaf((float)m[3], d.x, fmaf((float)m[4], d.y, (float)m[5] * d.z)),
+                    fmaf((float)m[6], d.x, fmaf((float)m[7], d.y, (float)m[8] * d.z)));
             co = mk((float)(m[0] * px + m[1] * py + m[2] * pz), (float)(m[3] * px + m[4] * py + m[5] * pz),
                     (float)(m[6] * px + m[7] * py + m[8] * pz));
           }
-          cd = mk(fmaf(r0.x, d.x, fmaf(r0.y, d.y, r0.z * d.z)), fmaf(r1.x, d.x, fmaf(r1.y, d.y, r1.z * d.z)),
-                  fmaf(r2.x, d.x, fmaf(r2.y, d.y, r2.z * d.z)));
           const float len = sqrtf(dot(cd, cd));
           lo = fmaxf(tmin, tmin / len) - shift;
           best_t -= shift;

@@ -31,9 +31,7 @@ static_assert(TPT_WF_BLOCK % 64 == 0 && TPT_WF_BLOCK / 64 <= 7, "block_slot keep
 #define TPT_CNT_IDX(q, g) (((q) * TPT_WF_SEGS + (g)) * TPT_CNT_STRIDE)
 #define TPT_CNT_ACTIVE (5 * TPT_WF_SEGS * TPT_CNT_STRIDE)    // adaptive active-pixel list (one dense queue)
 #define TPT_CNT_OVERFLOW (TPT_CNT_ACTIVE + TPT_CNT_STRIDE)  // set if a segment would overflow (never by construction)
-#define TPT_CNT_FETCH (TPT_CNT_OVERFLOW + TPT_CNT_STRIDE)    // next ray of the refilling extension kernel
-#define TPT_CNT_FETCH_SH(q) (TPT_CNT_FETCH + (1 + (q)) * TPT_CNT_STRIDE)  // next ray of shadow queue q (refilling)
-#define TPT_NUM_CNT (TPT_CNT_FETCH + 3 * TPT_CNT_STRIDE)
+#define TPT_NUM_CNT (TPT_CNT_OVERFLOW + TPT_CNT_STRIDE)
 #define TPT_STAT_STRIDE 32  // uint64 words of statistics per segment (256 B)
 #define TPT_STAT_WORDS (TPT_WF_SEGS * TPT_STAT_STRIDE)
 // Few paths: a bounce's four or five launches take 40 to 300 us however few paths they have (cold
@@ -106,7 +104,7 @@ struct QueueMap {
 #pragma unroll
     for (int g = 0; g < TPT_WF_SEGS; g++) {
       pre[g] = s;
-      s += counters[TPT_CNT_IDX(q, g)];
+      s += (uint32_t)__builtin_amdgcn_readfirstlane((int)counters[TPT_CNT_IDX(q, g)]);
     }
     n = s;
     cap = seg_cap;
@@ -158,9 +156,8 @@ struct WfParams {
   int32_t max_bounces, rr_start;
   float inv_w, inv_h;
   uint64_t seed;
-  int32_t refill;        // extension waves take new rays once fewer than this many lanes trace (0: one ray per lane)
-  int32_t refill_first;  // the same for the first bounce's extension (its camera rays)
-  int32_t refill_sh;     // the same for the shadow kernels
+  int32_t refill;  // persistent traversal after the first bounce: rays start once fewer than this many lanes of a
+                   // wave are tracing (0: one ray per lane)
   int32_t pad;
 };
 
