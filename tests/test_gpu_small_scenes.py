@@ -46,3 +46,19 @@ def test_small_scene_kernels_keep_the_image(gpu_ctx, name, w, h, spp):
         np.testing.assert_array_equal(getattr(a, f), getattr(b, f), err_msg=f)
     for k in ("rays_extension", "rays_shadow", "light_samples", "light_self_occluded"):
         assert a.stats[k] == b.stats[k], k
+
+
+@pytest.mark.parametrize("name", ["cornell", "1280_triangles"])
+@pytest.mark.parametrize("w,h,spp", [(513, 1, 512), (1, 300, 1024), (640, 360, 3), (1023, 513, 1)])
+def test_camera_rays_are_each_traced_once(gpu_ctx, name, w, h, spp):
+    """The order in which blocks take the camera rays, at widths and path counts around multiples of
+    a block and of the grid: every path is counted and traced once, and one pass sums what passes
+    of single samples (which go to the kernel that walks whole paths) sum."""
+    ds = T.DeviceScene(SCENES[name](), gpu_ctx)
+    kw = dict(width=w, height=h, spp=spp, max_bounces=3, rr_start=4, seed=3)
+    a = T.render(ds, T.RenderConfig(**kw))
+    b = T.render(ds, T.RenderConfig(samples_per_pass=min(spp, 512 if w == 1 else 1 if w < 1000 else spp),
+                                    traversal_refill=-1, **kw))
+    assert a.stats["paths"] == b.stats["paths"] == w * h * spp
+    assert a.stats["rays_extension"] == b.stats["rays_extension"]
+    np.testing.assert_allclose(a.acc, b.acc, rtol=1e-12, atol=0)  # FP64 sums of up to 1024 terms, grouped differently
