@@ -10,6 +10,7 @@ import pytest
 import tinypt_amd as T
 from parity_scenes import PARITY_CASES, floorlight
 from tinypt_amd import scenes
+from tinypt_amd.scene import DiffuseLight, Instance, Mesh, Transform
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +63,31 @@ def test_camera_rays_are_each_traced_once(gpu_ctx, name, w, h, spp):
     assert a.stats["paths"] == b.stats["paths"] == w * h * spp
     assert a.stats["rays_extension"] == b.stats["rays_extension"]
     np.testing.assert_allclose(a.acc, b.acc, rtol=1e-12, atol=0)  # FP64 sums of up to 1024 terms, grouped differently
+
+
+@pytest.mark.parametrize("bounces", [6, 12])
+@pytest.mark.parametrize("name", ["cornell", "spheres", "spheres_in_box", "zoo", "root_is_a_leaf", "80_triangles"])
+def test_short_passes_and_gradients_of_small_scenes(gpu_ctx, name, bounces):
+    """The kernel that walks whole paths and the adjoint read the trees from LDS too: the sums of a
+    short pass equal those of the device-memory form bit for bit, and the gradient that of the same
+    scene with 5120 triangles added far away, which make it a large one.  Both sum the same path
+    terms, a block at a time in FP32 and in another order: n = 1536 terms of a block give
+    sqrt(n) 2^-24 = 2.3e-6 of the sum of their magnitudes, 1e-4 of the largest gradient where a
+    fortieth of that sum is left; roughness differences cancel further, 1e-3."""
+    kw = dict(width=41, height=29, spp=12, max_bounces=bounces, rr_start=4, seed=5)
+    ds = T.DeviceScene(SCENES[name](), gpu_ctx)
+    few, plain = (T.render(ds, T.RenderConfig(traversal_refill=r, **kw)) for r in (0, -1))
+    for f in ("acc", "acc_w", "acc_sq"):
+        np.testing.assert_array_equal(getattr(few, f), getattr(plain, f), err_msg=f)
+    big = SCENES[name]()
+    speck = 1e-3 * scenes.displaced_icosphere(4)[0] + np.array([3e3, -9e3, 5e3])
+    dark = next(k for k, m in enumerate(big.mats) if m.kind != DiffuseLight((1, 1, 1)).kind)
+    big.world.meshes.append(Mesh(speck, dark))
+    big.world.instances.append(Instance(len(big.world.meshes) - 1, Transform.identity(), None))
+    dl = np.ones((29, 41, 3), np.float32)
+    g, _ = T.render_adjoint(ds, T.RenderConfig(**kw), dl)
+    h, _ = T.render_adjoint(T.DeviceScene(big, gpu_ctx), T.RenderConfig(**kw), dl)
+    g, h = np.asarray(g), np.asarray(h)
+    scale = np.abs(h).max()
+    np.testing.assert_allclose(g[:, :3], h[:, :3], rtol=0, atol=1e-4 * scale)
+    np.testing.assert_allclose(g[:, 3], h[:, 3], rtol=0, atol=1e-3 * scale)

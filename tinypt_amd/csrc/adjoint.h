@@ -7,6 +7,7 @@
 
 #include "../../include/tinypt_gpu.h"
 #include "tpt_kernels.h"
+#include "tpt_small32.h"
 #include "tpt_trace32.h"
 
 namespace tpt {
@@ -24,7 +25,7 @@ enum { ADJ_SCRATCH_DLDP, ADJ_SCRATCH_GRAD, ADJ_SCRATCH_STATS, ADJ_SCRATCH_APM, A
 // Bytes of each buffer of AdjScratch for a render of cfg over n_mats materials.
 void adjoint_scratch_bytes(const tpt_render_config* cfg, int n_mats, int stack_need, size_t bytes[ADJ_SCRATCH_N]);
 
-int adjoint_render(hipStream_t s, const SceneF32& S, const SceneF64& S64, const EnvDev& env, const LightsDev& lights, const MatsDev& mats,
+int adjoint_render(hipStream_t s, const SceneF32& S, const SmallScene& small, const SceneF64& S64, const EnvDev& env, const LightsDev& lights, const MatsDev& mats,
                    const CamF32& cam, const double* mat_param, int stack_need, const tpt_render_config* cfg,
                    const float* d_loss_d_pixel, double* grad_params, tpt_stats* stats, const AdjScratch& scratch,
                    std::string* err);

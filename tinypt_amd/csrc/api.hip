@@ -1133,7 +1133,7 @@ int tpt_render_adjoint(tpt_ctx* ctx, const tpt_scene* scene, const tpt_render_co
   }
   const AdjScratch scratch{p[ADJ_SCRATCH_DLDP], p[ADJ_SCRATCH_GRAD], p[ADJ_SCRATCH_STATS], p[ADJ_SCRATCH_APM],
                            p[ADJ_SCRATCH_GSTACK]};
-  return adjoint_render(ctx->stream, scene->s32, scene->s64, scene->env, scene->lights, scene->mats, scene->cam32,
+  return adjoint_render(ctx->stream, scene->s32, small_scene(scene->host, 0), scene->s64, scene->env, scene->lights, scene->mats, scene->cam32,
                         scene->host.mat_param.data(), stack_need(scene->host), cfg, d_loss_d_pixel, grad_params, stats,
                         scratch, &g_err);
 }

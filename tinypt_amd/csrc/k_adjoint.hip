@@ -73,6 +73,7 @@ struct GgxList {
 
 struct AdjParams {
   SceneF32 S;
+  SmallScene small;
   SceneF64 S64;  // reference-layout scene, for the light self-occlusion decision
   EnvDev env;
   LightsDev lights;
@@ -138,8 +139,8 @@ __device__ __forceinline__ void add_suffix_terms(GradSink& sink, int mat, f3 num
 // The mode is a run-time value, so the kernel holds one inlined copy of the replay: a copy per
 // mode took 256 VGPRs plus 620 B of private memory per lane and ran one wave per SIMD; one copy
 // runs three waves per SIMD (168 VGPRs, some spilled) and the kernel 2.3x faster.
-template <bool ENV_NEE, class Stack>
-__device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, uint32_t x, uint32_t y, uint32_t s, f3 delta,
+template <bool ENV_NEE, class Tree, class Stack>
+__device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, const Tree& tree, uint32_t x, uint32_t y, uint32_t s, f3 delta,
                                      f3 S_total, GradSink& sink, GgxList* ggx, VertexLog* log, int pert_mat,
                                      float pert_alpha, const Stack& st, uint32_t* n_ext, uint32_t* n_sh) {
   const bool GRAD = MODE == ADJ_GRAD || MODE == ADJ_SUMGRAD;
@@ -152,7 +153,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, uint32_
   for (int bounce = 0; bounce < A.max_bounces; bounce++) {
     HitF32 h;
     (*n_ext)++;
-    if (!trace_f32<false>(A.S, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st)) {
+    if (!trace_f32<false>(A.S, tree, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st)) {
       // miss (integrator.rs:71-83)
       f3 bg = A.env.black ? mk(0.f, 0.f, 0.f) : (ENV_NEE ? env_lookup32(A.env, d) : sky32(d));
       f3 x0 = had(T, bg);
@@ -208,7 +209,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, uint32_
           if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
             HitF32 hs;
             (*n_sh)++;
-            if (!trace_f32<true>(A.S, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, 1e30f, &hs, st)) {
+            if (!trace_f32<true>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, 1e30f, &hs, st)) {
               S_upto = S_upto + had(c, delta);
               if (GRAD) {
                 f3 base = had(had(T, li), delta) * (cs / pe);  // dc_c/df_c * delta_c / w
@@ -246,7 +247,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, uint32_
               float tmax = light_shadow_tmax32(dist);
               HitF32 hs;
               (*n_sh)++;
-              if (!trace_f32<true>(A.S, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, tmax, &hs, st)) {
+              if (!trace_f32<true>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, tmax, &hs, st)) {
                 S_upto = S_upto + had(c, delta);
                 if (GRAD) {
                   f3 base = had(had(T, ls.emit), delta) * (cs / ls.pdf);
@@ -348,8 +349,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // material by material: the FP32 sums of a block keep their order.  i: this lane's path; every lane
 // of the wave must call it.  Short paths do without: their lane-by-lane sums are repeated to 1e-8, and
 // this changes the order in which a block's waves add.
-template <bool ENV_NEE, class Stack>
-__device__ __forceinline__ void replay_items(const AdjParams& A, uint64_t i, const GgxList& ggx, uint2* items,
+template <bool ENV_NEE, class Tree, class Stack>
+__device__ __forceinline__ void replay_items(const AdjParams& A, const Tree& tree, uint64_t i, const GgxList& ggx, uint2* items,
                                              GradSink& sink, const Stack& st, uint32_t* n_ext, uint32_t* n_sh) {
   const uint32_t lane = __lane_id();
   const uint64_t below = (1ull << lane) - 1ull;
@@ -370,7 +371,7 @@ __device__ __forceinline__ void replay_items(const AdjParams& A, uint64_t i, con
         const uint2 it = items[j];
         const AdjPath q = adj_path(A, i - lane + it.x);
         const int m = (int)it.y;
-        const f3 v = replay<ENV_NEE>(ADJ_VALUE, A, q.x, q.y, q.s, q.delta, mk(0.f, 0.f, 0.f), sink, nullptr, nullptr, m,
+        const f3 v = replay<ENV_NEE>(ADJ_VALUE, A, tree, q.x, q.y, q.s, q.delta, mk(0.f, 0.f, 0.f), sink, nullptr, nullptr, m,
                                      A.alpha_pm[2 * m + (lane & 1)], st, n_ext, n_sh);
         const f3 w = mk(__shfl_xor(v.x, 1), __shfl_xor(v.y, 1), __shfl_xor(v.z, 1));
         if ((lane & 1) == 0) {  // loss term at alpha + h minus the one at alpha - h
@@ -391,18 +392,28 @@ __device__ __forceinline__ void replay_items(const AdjParams& A, uint64_t i, con
   }
 }
 
-// OVF: the traversal stack may overflow to global memory; ENV_NEE: the environment takes part in
-// next-event estimation; ONE: paths short enough to log (one replay for sums and gradients).
-template <bool OVF, bool ENV_NEE, bool ONE>
+// Tree: GlobalTree, or SmallTree for small scenes (tpt_small32.h): replays are bound by the latency of
+// a few waves per SIMD, and node loads from LDS shorten it (inverse step of 16 spheres in the Cornell
+// box, 256^2 x 16 spp: 5.3 -> 4.75 ms).  OVF: the traversal stack may overflow to global memory;
+// ENV_NEE: the environment takes part in next-event estimation; ONE: paths short enough to log (one replay for sums and gradients).
+template <class Tree, bool OVF, bool ENV_NEE, bool ONE>
 __global__ void __launch_bounds__(TPT_ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(3))) k_adjoint(AdjParams A) {
-  __shared__ int32_t s_stack[TPT_WF_STACK_ADJ * TPT_ADJ_BLOCK];
+  extern __shared__ float4 s_trees[];  // the lanes' stacks, and a small scene's trees
   __shared__ float s_grad[TPT_ADJ_LDS_GRAD];
   __shared__ uint2 s_items[ONE ? 1 : TPT_ADJ_BLOCK / 64 * TPT_ADJ_ITEMS];
   for (int i = threadIdx.x; i < TPT_ADJ_LDS_GRAD; i += blockDim.x) s_grad[i] = 0.f;
   __syncthreads();
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? A.gstack + gid * (uint64_t)A.gcap : nullptr, TPT_ADJ_BLOCK,
-                     TPT_WF_STACK_ADJ};
+  LaneStackT<OVF> st;
+  const Tree tree = [&] {
+    if constexpr (Tree::kWorldOnly) {
+      return load_small<TPT_ADJ_BLOCK>(A.S, A.small, s_trees, &st);
+    } else {
+      st = LaneStackT<OVF>{reinterpret_cast<int32_t*>(s_trees) + threadIdx.x,
+                           OVF ? A.gstack + gid * (uint64_t)A.gcap : nullptr, TPT_ADJ_BLOCK, TPT_WF_STACK_ADJ};
+      return GlobalTree{A.S};
+    }
+  }();
   GradSink sink{s_grad, A.grad, A.n_mats};
   uint32_t n_ext = 0, n_sh = 0, n_paths = 0;
   const f3 zero = mk(0.f, 0.f, 0.f);
@@ -421,7 +432,7 @@ __global__ void __launch_bounds__(TPT_ADJ_BLOCK) __attribute__((amdgpu_waves_per
         const int vi = pass - 1;
         const int m = vi >= 0 ? ggx.mat[vi >> 1] : -1;
         const float alpha = vi >= 0 ? A.alpha_pm[2 * m + (vi & 1)] : 0.f;
-        const f3 v = replay<ENV_NEE>(pass == 0 ? ADJ_SUMGRAD : ADJ_VALUE, A, q.x, q.y, q.s, q.delta, zero, sink,
+        const f3 v = replay<ENV_NEE>(pass == 0 ? ADJ_SUMGRAD : ADJ_VALUE, A, tree, q.x, q.y, q.s, q.delta, zero, sink,
                                      pass == 0 ? &ggx : nullptr, pass == 0 ? &log : nullptr, m, alpha, st, &n_ext, &n_sh);
         if (pass == 0) {
           for (int j = 0; j < log.n; j++) add_suffix_terms(sink, log.mat[j], log.num[j], log.den[j], v - log.s_upto[j]);
@@ -444,11 +455,11 @@ __global__ void __launch_bounds__(TPT_ADJ_BLOCK) __attribute__((amdgpu_waves_per
         // pass 0 sums the path's terms (and lists its GGX materials), pass 1 takes the gradients
         f3 S_total = zero;
         for (int pass = 0; pass < 2; pass++)
-          S_total = replay<ENV_NEE>(pass == 0 ? ADJ_SUM : ADJ_GRAD, A, q.x, q.y, q.s, q.delta, S_total, sink,
+          S_total = replay<ENV_NEE>(pass == 0 ? ADJ_SUM : ADJ_GRAD, A, tree, q.x, q.y, q.s, q.delta, S_total, sink,
                                     pass == 0 ? &ggx : nullptr, nullptr, -1, 0.f, st, &n_ext, &n_sh);
         n_paths++;
       }
-      replay_items<ENV_NEE>(A, i, ggx, s_items + (threadIdx.x >> 6) * TPT_ADJ_ITEMS, sink, st, &n_ext, &n_sh);
+      replay_items<ENV_NEE>(A, tree, i, ggx, s_items + (threadIdx.x >> 6) * TPT_ADJ_ITEMS, sink, st, &n_ext, &n_sh);
     }
   }
   __syncthreads();
@@ -482,7 +493,7 @@ void adjoint_scratch_bytes(const tpt_render_config* cfg, int n_mats, int stack_n
   bytes[ADJ_SCRATCH_GSTACK] = gcap > 0 ? (size_t)adjoint_blocks(n_paths) * TPT_ADJ_BLOCK * gcap * 4 : 0;
 }
 
-int adjoint_render(hipStream_t s, const SceneF32& S, const SceneF64& S64, const EnvDev& env, const LightsDev& lights, const MatsDev& mats,
+int adjoint_render(hipStream_t s, const SceneF32& S, const SmallScene& small, const SceneF64& S64, const EnvDev& env, const LightsDev& lights, const MatsDev& mats,
                    const CamF32& cam, const double* mat_param, int stack_need, const tpt_render_config* cfg,
                    const float* d_loss_d_pixel, double* grad_params, tpt_stats* stats, const AdjScratch& scratch,
                    std::string* err) {
@@ -509,6 +520,7 @@ int adjoint_render(hipStream_t s, const SceneF32& S, const SceneF64& S64, const 
   if (e != hipSuccess) return fail(TPT_ERR_DEVICE, std::string("adjoint setup: ") + hipGetErrorString(e));
   AdjParams A{};
   A.S = S;
+  A.small = small;
   A.S64 = S64;
   A.env = env;
   A.lights = lights;
@@ -536,14 +548,18 @@ int adjoint_render(hipStream_t s, const SceneF32& S, const SceneF64& S64, const 
   (void)hipEventRecord(e0, s);
   const bool env_nee = env.kind == TPT_ENV_IMAGE && !env.black;
   const bool one = cfg->max_bounces <= TPT_ADJ_LOG + 1;  // at most max_bounces - 1 BSDF vertices
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(TPT_ADJ_BLOCK), 0, s, A); };
+  const uint32_t lds = small.bytes > 0 ? small_lds(small, TPT_ADJ_BLOCK) : TPT_WF_STACK_ADJ * TPT_ADJ_BLOCK * 4;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(TPT_ADJ_BLOCK), lds, s, A); };
   if (n_paths > 0) {
-    if (gcap > 0) {
-      if (env_nee) one ? launch(k_adjoint<true, true, true>) : launch(k_adjoint<true, true, false>);
-      else one ? launch(k_adjoint<true, false, true>) : launch(k_adjoint<true, false, false>);
+    if (small.bytes > 0) {
+      if (env_nee) one ? launch(k_adjoint<SmallTree, false, true, true>) : launch(k_adjoint<SmallTree, false, true, false>);
+      else one ? launch(k_adjoint<SmallTree, false, false, true>) : launch(k_adjoint<SmallTree, false, false, false>);
+    } else if (gcap > 0) {
+      if (env_nee) one ? launch(k_adjoint<GlobalTree, true, true, true>) : launch(k_adjoint<GlobalTree, true, true, false>);
+      else one ? launch(k_adjoint<GlobalTree, true, false, true>) : launch(k_adjoint<GlobalTree, true, false, false>);
     } else {
-      if (env_nee) one ? launch(k_adjoint<false, true, true>) : launch(k_adjoint<false, true, false>);
-      else one ? launch(k_adjoint<false, false, true>) : launch(k_adjoint<false, false, false>);
+      if (env_nee) one ? launch(k_adjoint<GlobalTree, false, true, true>) : launch(k_adjoint<GlobalTree, false, true, false>);
+      else one ? launch(k_adjoint<GlobalTree, false, false, true>) : launch(k_adjoint<GlobalTree, false, false, false>);
     }
   }
   e = hipGetLastError();

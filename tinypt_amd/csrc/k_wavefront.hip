@@ -180,50 +180,7 @@ k_extend(WfParams W, int cur, PassArgs A, PathCount count) {
   }
 }
 
-// ---------------------------------------------------------------- small scenes: trees in LDS
-// (measurements at k_extend_small)
-struct SmallTree {
-  static constexpr bool kWorldOnly = true;
-  const char *nodes, *tris, *sph;  // LDS, offset so that the scene's own indices address them
-  const int32_t *inst, *items;
-  int32_t root;
-  __device__ __forceinline__ uint32_t node(int32_t ref) const { return (uint32_t)ref * TPT_SMALL_NODE_BYTES; }
-  __device__ __forceinline__ float4 planes(uint32_t at) const { return *reinterpret_cast<const float4*>(nodes + (int32_t)at); }
-  __device__ __forceinline__ int4 children(uint32_t at) const {
-    return *reinterpret_cast<const int4*>(nodes + (int32_t)(at + 96u));
-  }
-  __device__ __forceinline__ const float4* tri(uint32_t slot) const {
-    return reinterpret_cast<const float4*>(tris + (int32_t)(slot * 48u));
-  }
-  __device__ __forceinline__ int32_t tri_inst(uint32_t slot) const { return inst[(int32_t)slot]; }
-  __device__ __forceinline__ int32_t item(uint32_t k) const { return items[k]; }
-  __device__ __forceinline__ const double* sphere(int32_t s) const { return reinterpret_cast<const double*>(sph + s * 32); }
-  __device__ __forceinline__ int32_t flat_root() const { return root; }
-};
-
-// Copies the scene into `mem` (every thread of the block must call it) and returns its trees and, in
-// *stack, this lane's stack behind them.
-__device__ __forceinline__ SmallTree load_small(const SceneF32& S, const SmallScene& m, float4* mem, LaneStackT<false>* stack) {
-  float4* tris = mem + m.n_nodes * (TPT_SMALL_NODE_BYTES / 16);
-  float4* sph = tris + m.n_tris * 3;
-  int32_t* inst = reinterpret_cast<int32_t*>(sph + m.n_sph * 2);
-  int32_t* items = inst + m.n_tris;
-  const float4* gn = reinterpret_cast<const float4*>(S.nodes + m.node0);
-  for (uint32_t i = threadIdx.x; i < m.n_nodes * 7; i += TPT_WF_BLOCK) mem[i] = gn[i / 7 * 8 + i % 7];
-  const float4* gt = reinterpret_cast<const float4*>(S.tris + m.tri0);
-  for (uint32_t i = threadIdx.x; i < m.n_tris * 3; i += TPT_WF_BLOCK) tris[i] = gt[i];
-  const float4* gs = reinterpret_cast<const float4*>(S.sph);
-  for (uint32_t i = threadIdx.x; i < m.n_sph * 2; i += TPT_WF_BLOCK) sph[i] = gs[i];
-  for (uint32_t i = threadIdx.x; i < m.n_tris; i += TPT_WF_BLOCK) inst[i] = S.tri_inst[m.tri0 + i];
-  for (uint32_t i = threadIdx.x; i < m.n_items; i += TPT_WF_BLOCK) items[i] = S.tlas_items[i];
-  __syncthreads();
-  *stack = LaneStackT<false>{reinterpret_cast<int32_t*>(mem + m.bytes / 16) + threadIdx.x, nullptr, TPT_WF_BLOCK,
-                             (int)m.stack};
-  return SmallTree{reinterpret_cast<const char*>(mem) - m.node0 * TPT_SMALL_NODE_BYTES,
-                   reinterpret_cast<const char*>(tris) - m.tri0 * 48u, reinterpret_cast<const char*>(sph),
-                   inst - m.tri0, items, m.flat_root};
-}
-
+// ---------------------------------------------------------------- small scenes (tpt_small32.h)
 // A wave of k_extend_small / k_shadow_small starts rays once fewer lanes than this are tracing.
 #define TPT_SMALL_LANES 25
 #define TPT_SMALL_LANES_SH 17
@@ -314,7 +271,7 @@ k_extend_small(WfParams W, int cur, PassArgs A, PathCount count) {
     n = qm.n;
   }
   LaneStackT<false> st;
-  const SmallTree tree = load_small(W.S, W.small, s_small, &st);
+  const SmallTree tree = load_small<TPT_WF_BLOCK>(W.S, W.small, s_small, &st);
   begin_extension<GEN>(W, cur, n, count);
   if constexpr (GEN) {
     for (CameraTurns turn; turn.any(n); turn.next()) {
@@ -762,7 +719,7 @@ k_shadow_small(WfParams W, int queue, PathCount count) {
   extern __shared__ float4 s_small[];
   tell_count(W, count);
   LaneStackT<false> st;
-  const SmallTree tree = load_small(W.S, W.small, s_small, &st);
+  const SmallTree tree = load_small<TPT_WF_BLOCK>(W.S, W.small, s_small, &st);
   shadow_share(W, queue, tree, st, TPT_SMALL_LANES_SH);
 }
 
@@ -777,15 +734,30 @@ k_shadow_refill(WfParams W, int queue, PathCount count) {
   shadow_share(W, queue, GlobalTree{W.S}, st, W.refill);
 }
 
+// The trees k_tail walks and this lane's stack, in `mem`.
+template <class Tree, bool OVF>
+__device__ __forceinline__ Tree tail_tree(const WfParams& W, float4* mem, LaneStackT<OVF>* st) {
+  if constexpr (Tree::kWorldOnly) {
+    return load_small<TPT_WF_BLOCK>(W.S, W.small, mem, st);
+  } else {
+    *st = LaneStackT<OVF>{reinterpret_cast<int32_t*>(mem) + threadIdx.x,
+                          OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK, TPT_WF_STACK};
+    return GlobalTree{W.S};
+  }
+}
+
 // The rest of a few paths in one launch: each lane walks its path to the end -- extension, shading,
 // the light self-occlusion decision, shadow rays and scattering by the same functions as the
 // kernels above, contributions added in their order, so a path's radiance is the same bit for bit.
-// GEN: the whole paths of a small pass (camera rays generated here); otherwise the paths of queue
-// cur, whose hits this bounce's extension has stored.
-template <bool OVF, bool ENV_NEE, bool GEN>
+// Tree: SmallTree for small scenes (64^2 x 4 spp of the Cornell box 245 -> 233 us per render, the same
+// rays on device memory).  GEN: the whole paths of a small pass (camera rays generated here);
+// otherwise the paths of queue cur, whose hits this bounce's extension has stored.
+template <class Tree, bool OVF, bool ENV_NEE, bool GEN>
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
 k_tail(WfParams W, int cur, PassArgs A) {
-  __shared__ int32_t s_stack[TPT_WF_STACK * TPT_WF_BLOCK];
+  extern __shared__ float4 s_small[];
+  LaneStackT<OVF> st;
+  const Tree tree = tail_tree<Tree>(W, s_small, &st);
   QueueMap qm;
   uint32_t n;
   if constexpr (GEN) {
@@ -794,8 +766,6 @@ k_tail(WfParams W, int cur, PassArgs A) {
     qm.load(W.ps.counters, cur ? TPT_CNT_Q1 : TPT_CNT_Q0, W.ps.seg_cap);
     n = qm.n;
   }
-  LaneStackT<OVF> st{s_stack + threadIdx.x, OVF ? W.gstack + (size_t)gtid() * W.gstack_cap : nullptr, TPT_WF_BLOCK,
-                     TPT_WF_STACK};
   const uint32_t lanes = lanes_per_wave(n);
   uint32_t next = (gtid() >> 6) * lanes + __lane_id();
   if (__lane_id() >= lanes) next = n;
@@ -827,7 +797,7 @@ k_tail(WfParams W, int cur, PassArgs A) {
     }
     if (!have_hit) {
       HitF32 t;
-      trace_f32<false>(W.S, v.o, v.d, (float)TPT_RAY_EPSILON, 1e30f, &t, st);
+      trace_f32<false>(W.S, tree, v.o, v.d, (float)TPT_RAY_EPSILON, 1e30f, &t, st);
       h = HitRec{__float_as_int(t.t), t.inst, t.prim};
       n_ext++;
     }
@@ -847,7 +817,7 @@ k_tail(WfParams W, int cur, PassArgs A) {
       } else {
         HitF32 t;
         n_sh++;
-        if (!trace_f32<true>(W.S, sf.p + (float)TPT_RAY_EPSILON * nee.l_d, nee.l_d, (float)TPT_RAY_EPSILON,
+        if (!trace_f32<true>(W.S, tree, sf.p + (float)TPT_RAY_EPSILON * nee.l_d, nee.l_d, (float)TPT_RAY_EPSILON,
                              light_shadow_tmax32(nee.l_dist), &t, st))
           L = L + nee.l_c;
       }
@@ -855,7 +825,7 @@ k_tail(WfParams W, int cur, PassArgs A) {
     if (ENV_NEE && nee.env) {  // k_shadow on the environment queue
       HitF32 t;
       n_sh++;
-      if (!trace_f32<true>(W.S, nee.env_o, nee.env_d, (float)TPT_RAY_EPSILON, 1e30f, &t, st)) L = L + nee.env_c;
+      if (!trace_f32<true>(W.S, tree, nee.env_o, nee.env_d, (float)TPT_RAY_EPSILON, 1e30f, &t, st)) L = L + nee.env_c;
     }
     alive = alive && scatter_vertex(W, sf, v);
     if (!alive) W.ps.L[id] = make_float4(L.x, L.y, L.z, 0.f);
@@ -993,8 +963,7 @@ static uint32_t resident_blocks(const void* kernel, uint32_t lds = 0) {
 static inline dim3 grid_of(uint32_t n, const void* kernel, uint32_t lds = 0) {
   return dim3(std::min(grid_for(n), resident_blocks(kernel, lds)));
 }
-// LDS of the small-scene kernels: the scene and the lanes' stacks.
-static inline uint32_t small_lds(const WfParams& W) { return W.small.bytes + W.small.stack * TPT_WF_BLOCK * 4; }
+static inline uint32_t small_lds(const WfParams& W) { return small_lds(W.small, TPT_WF_BLOCK); }
 
 hipError_t wf_launch_clear_radiance(const WfParams& W, uint32_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_clear_radiance, dim3(grid_for(n)), dim3(TPT_WF_BLOCK), 0, s, W, n);
@@ -1024,21 +993,27 @@ hipError_t wf_launch_extend(const WfParams& W, int cur, const PassArgs* gen, con
   }
   return hipGetLastError();
 }
-template <bool OVF, bool ENV_NEE>
+template <class Tree, bool OVF, bool ENV_NEE>
 static void launch_tail(const WfParams& W, int cur, const PassArgs* gen, uint32_t n, hipStream_t s) {
   const PassArgs A = gen ? *gen : PassArgs{};
+  const uint32_t lds = Tree::kWorldOnly ? small_lds(W) : TPT_WF_STACK * TPT_WF_BLOCK * 4;
   auto launch = [&](auto kernel) {
     const uint32_t waves = (n + TPT_WF_MIN_LANES - 1) / TPT_WF_MIN_LANES;
-    hipLaunchKernelGGL(kernel, grid_of(std::min(waves, 1u << 20) * 64, (const void*)kernel), dim3(TPT_WF_BLOCK), 0, s, W,
-                       cur, A);
+    hipLaunchKernelGGL(kernel, grid_of(std::min(waves, 1u << 20) * 64, (const void*)kernel, lds), dim3(TPT_WF_BLOCK), lds,
+                       s, W, cur, A);
   };
-  if (gen) launch(k_tail<OVF, ENV_NEE, true>);
-  else launch(k_tail<OVF, ENV_NEE, false>);
+  if (gen) launch(k_tail<Tree, OVF, ENV_NEE, true>);
+  else launch(k_tail<Tree, OVF, ENV_NEE, false>);
 }
 static inline bool env_nee(const WfParams& W) { return W.env.kind == TPT_ENV_IMAGE && !W.env.black; }
 hipError_t wf_launch_tail(const WfParams& W, int cur, const PassArgs* gen, uint32_t n, hipStream_t s) {
-  if (W.gstack) env_nee(W) ? launch_tail<true, true>(W, cur, gen, n, s) : launch_tail<true, false>(W, cur, gen, n, s);
-  else env_nee(W) ? launch_tail<false, true>(W, cur, gen, n, s) : launch_tail<false, false>(W, cur, gen, n, s);
+  const bool env = env_nee(W);
+  if (W.small.bytes > 0)
+    env ? launch_tail<SmallTree, false, true>(W, cur, gen, n, s) : launch_tail<SmallTree, false, false>(W, cur, gen, n, s);
+  else if (W.gstack)
+    env ? launch_tail<GlobalTree, true, true>(W, cur, gen, n, s) : launch_tail<GlobalTree, true, false>(W, cur, gen, n, s);
+  else
+    env ? launch_tail<GlobalTree, false, true>(W, cur, gen, n, s) : launch_tail<GlobalTree, false, false>(W, cur, gen, n, s);
   return hipGetLastError();
 }
 template <bool ENV_NEE, bool GEN>
