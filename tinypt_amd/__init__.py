@@ -231,10 +231,10 @@ class DeviceScene(_SceneTables):
         """FP32 closest hit (World::hit semantics).  rays (n, 8): o, d, tmin, tmax."""
         r = np.ascontiguousarray(np.asarray(rays, dtype=np.float32).reshape(-1, 8))
         n = len(r)
-        t = np.zeros(n, np.float32)
-        kind = np.zeros(n, np.int32)
-        inst = np.zeros(n, np.int32)
-        prim = np.zeros(n, np.int32)
+        # one block: from 4 MB on numpy asks for huge pages, and most of the time of filling fresh
+        # arrays goes into their page faults
+        out = np.empty((4, n), np.int32)
+        t, kind, inst, prim = out[0].view(np.float32), out[1], out[2], out[3]
         ip = lambda a: a.ctypes.data_as(C.POINTER(C.c_int32))
         _check(self._lib.tpt_trace_closest(self.ctx.h, self.h, n, r.ctypes.data_as(C.POINTER(C.c_float)),
                                            t.ctypes.data_as(C.POINTER(C.c_float)), ip(kind), ip(inst), ip(prim)))
