@@ -111,10 +111,10 @@ def measured_valu():
     if not os.path.exists(path):
         return None
     for line in open(path):
-        if line.startswith("| `void tpt::k_extend<false, false>"):
+        if line.startswith("| `void tpt::k_extend_small<false>"):
             cols = [c.strip() for c in line.strip().strip("|").split("|")]
-            return {"valu_busy_pct": float(cols[3]), "valu_lane_utilisation_pct": float(cols[4]),
-                    "occupancy_pct": float(cols[5]), "source": VALU_PROFILE}
+            return {"valu_busy_pct": float(cols[2]), "valu_lane_utilisation_pct": float(cols[3]),
+                    "occupancy_pct": float(cols[4]), "source": VALU_PROFILE}
     return None
 
 
