@@ -153,7 +153,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, const T
   for (int bounce = 0; bounce < A.max_bounces; bounce++) {
     HitF32 h;
     (*n_ext)++;
-    if (!trace_f32<false>(A.S, tree, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st)) {
+    if (!trace_f32<false, false>(A.S, tree, o, d, (float)TPT_RAY_EPSILON, 1e30f, &h, st)) {
       // miss (integrator.rs:71-83)
       f3 bg = A.env.black ? mk(0.f, 0.f, 0.f) : (ENV_NEE ? env_lookup32(A.env, d) : sky32(d));
       f3 x0 = had(T, bg);
@@ -209,7 +209,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, const T
           if (c.x != 0.f || c.y != 0.f || c.z != 0.f) {
             HitF32 hs;
             (*n_sh)++;
-            if (!trace_f32<true>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, 1e30f, &hs, st)) {
+            if (!trace_f32<true, false>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, 1e30f, &hs, st)) {
               S_upto = S_upto + had(c, delta);
               if (GRAD) {
                 f3 base = had(had(T, li), delta) * (cs / pe);  // dc_c/df_c * delta_c / w
@@ -247,7 +247,7 @@ __device__ __forceinline__ f3 replay(const int MODE, const AdjParams& A, const T
               float tmax = light_shadow_tmax32(dist);
               HitF32 hs;
               (*n_sh)++;
-              if (!trace_f32<true>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, tmax, &hs, st)) {
+              if (!trace_f32<true, false>(A.S, tree, p + (float)TPT_RAY_EPSILON * wi, wi, (float)TPT_RAY_EPSILON, tmax, &hs, st)) {
                 S_upto = S_upto + had(c, delta);
                 if (GRAD) {
                   f3 base = had(had(T, ls.emit), delta) * (cs / ls.pdf);
@@ -345,10 +345,12 @@ __device__ __forceinline__ void wave_lds_sync() {
 // item, one replaying the path at +h and one at -h (nearly the same path, side by side).  A path
 // meets few GGX materials and most meet none, so replaying them lane by lane -- two passes for
 // every material of the wave's richest path -- left most lanes idle (12-bounce paths over 20 mesh
-// materials, 128^2 x 16 spp: 3.16 -> 2.50 ms).  Each difference is added by the lane whose path it is,
-// material by material: the FP32 sums of a block keep their order.  i: this lane's path; every lane
-// of the wave must call it.  Short paths do without: their lane-by-lane sums are repeated to 1e-8, and
-// this changes the order in which a block's waves add.
+// materials, 128^2 x 16 spp: 3.16 -> 2.55 ms).  Each difference is added by the lane whose path it
+// is, material by material, so a wave adds its terms in the order of the lane-by-lane form; the
+// waves of a block add in FP32 in the order in which they come, as they did, which is what two runs
+// differ by (1e-8 to 1e-7 of the gradient's norm).  i: this lane's path; every lane of the wave must
+// call it.  Short paths do without: their sums repeat to 1e-9 in part, and adding a wave's roughness
+// terms in one burst moves them further than that.
 template <bool ENV_NEE, class Tree, class Stack>
 __device__ __forceinline__ void replay_items(const AdjParams& A, const Tree& tree, uint64_t i, const GgxList& ggx, uint2* items,
                                              GradSink& sink, const Stack& st, uint32_t* n_ext, uint32_t* n_sh) {

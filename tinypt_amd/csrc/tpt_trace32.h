@@ -184,7 +184,13 @@ struct GlobalTree {
 // 32 spp 39.6 -> 36.7 ms, 4096 instances adaptive 51.7 -> 46.9, Cornell box 512^2 x 256 spp
 // 27.75 -> 27.1; two eighths 37.0, 46.6, 27.2; four 36.7, 47.4, 27.1; five 37.2, 48.5, 27.3; to
 // the last lane 42.3, 47.2, 27.7.
-template <bool ANY, class Tree = GlobalTree>
+// VOTE = false, for the adjoint: every lane goes to its leaf before any leaf is handled and pops
+// after the leaves.  The waves of a block add their gradient terms in FP32 in the order in which
+// they come to them; with the vote they come in another order, and gradients of small renders
+// moved by up to 1.5e-7 of their norm, four times what two runs differ by.  Without it they stay
+// within that.  It costs 12-bounce gradients over 20 mesh materials 2.36 -> 2.55 ms (128^2 x 16
+// spp) and the inverse step of 16 spheres 4.60 -> 4.63 (256^2 x 16 spp).
+template <bool ANY, class Tree = GlobalTree, bool VOTE = true>
 struct TraceF32 {
   vec3<float> o, d;        // world ray
   vec3<float> co, cd;      // ray of the current level (object space inside an instance; unused if kWorldOnly)
@@ -258,11 +264,16 @@ struct TraceF32 {
     constexpr bool kWorld = Tree::kWorldOnly;
     // ---- descend inner nodes: four child boxes from one 128 B node; the nearest hit child
     // is entered, the others are pushed farthest first
+    bool have = true;
     for (;;) {
 #ifdef __HIP_DEVICE_COMPILE__
-      const bool node = at_node();
-      if (8 * __popcll(__ballot(node)) < TPT_NODE_LANES * __popcll(__ballot(true))) break;
-      if (!node) continue;
+      if constexpr (VOTE) {
+        const bool node = at_node();
+        if (8 * __popcll(__ballot(node)) < TPT_NODE_LANES * __popcll(__ballot(true))) break;
+        if (!node) continue;
+      } else {
+        if (!at_node()) break;
+      }
 #else
       if (!at_node()) break;
 #endif
@@ -290,6 +301,10 @@ struct TraceF32 {
         nhit += h ? 1 : 0;
       }
       if (nhit == 0) {
+        if constexpr (!VOTE) {
+          have = false;
+          break;
+        }
         if (!next(st)) return false;
         continue;
       }
@@ -323,8 +338,9 @@ struct TraceF32 {
       ref = cr[0];
     }
 #ifdef __HIP_DEVICE_COMPILE__
-    if (at_node()) return true;  // waits for the wave's leaves
+    if (VOTE && at_node()) return true;  // waits for the wave's leaves
 #endif
+    if (!VOTE && !have) return next(st);  // no child was hit
     if (ref == TPT_STACK_SENTINEL) {
       // ---- leaving an instance: back to the world ray (best_t back in world units: it is the
       // best hit's distance, or the ray's tmax while nothing is hit)
@@ -440,10 +456,10 @@ struct TraceF32 {
 };
 
 // Returns true on a hit.  ANY: stop at the first hit in range (shadow rays).
-template <bool ANY, class Tree, class Stack>
+template <bool ANY, bool VOTE = true, class Tree, class Stack>
 TPT_HD bool trace_f32(const SceneF32& S, const Tree& tree, vec3<float> o, vec3<float> d, float tmin, float tmax,
                       HitF32* hit, const Stack& st) {
-  TraceF32<ANY, Tree> tr;
+  TraceF32<ANY, Tree, VOTE> tr;
   if (tr.init(S, o, d, tmin, tmax)) {
     while (tr.step(S, st, tree)) {
     }
