@@ -942,7 +942,7 @@ int render_plain(tpt_ctx* c, const tpt_scene* sc, const tpt_render_config* cfg, 
   P.welford = c->welford.as<double>();
   P.done = c->done.as<uint8_t>();
   P.stats = c->stats.as<uint64_t>();
-  plain64_shape(sc->host.max_blas_depth, &P);
+  P.shape = plain64_shape(sc->host.max_blas_depth, P.n_pix);
   EventTimer total(s, st != nullptr, &c->ev_total);
   HIPC(total.mark());
   // samples of a launch: about 4M paths (a launch ends with its slowest pixel), at least 8

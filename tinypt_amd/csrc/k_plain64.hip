@@ -247,13 +247,13 @@ __device__ __forceinline__ bool world_hit(const Plain64Params& P, d3 o, d3 d, do
     float slack = 0.f;
     for (; ii < S.n_inst; ii++) {
       const float* b = P.inst_box + 6 * ii;
-    slack = 2e-6f * (o_max + fmaxf(fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))),
-                                               fmaxf(fabsf(b[4]), fabsf(b[5]))));
-    const float x0 = (b[0] - slack - ox) * ix, x1 = (b[3] + slack - ox) * ix;
-    const float y0 = (b[1] - slack - oy) * iy, y1 = (b[4] + slack - oy) * iy;
-    const float z0 = (b[2] - slack - oz) * iz, z1 = (b[5] + slack - oz) * iz;
-    const float in = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fminf(z0, z1));
-    const float out = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1));
+      slack = 2e-6f * (o_max + fmaxf(fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))),
+                                                 fmaxf(fabsf(b[4]), fabsf(b[5]))));
+      const float x0 = (b[0] - slack - ox) * ix, x1 = (b[3] + slack - ox) * ix;
+      const float y0 = (b[1] - slack - oy) * iy, y1 = (b[4] + slack - oy) * iy;
+      const float z0 = (b[2] - slack - oz) * iz, z1 = (b[5] + slack - oz) * iz;
+      const float in = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fminf(z0, z1));
+      const float out = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1));
       if (!(slack < 1e30f && (in > out || out < 0.f || in > (float)closest * 1.000002f + slack))) break;
     }
     if (ii >= S.n_inst) break;
@@ -561,7 +561,7 @@ __device__ __forceinline__ void vertex64(const Plain64Params& P, Path64& q, bool
 
 // ---------------------------------------------------------------- render.rs:137-191
 // A pixel's samples share one random stream, so a lane works through its pixel's samples in
-// order, taking the next sample as soon as a path ends.  G lanes per pixel (1 or 4), P.lanes lanes of
+// order, taking the next sample as soon as a path ends.  G lanes per pixel (1 or 4), P.shape.lanes lanes of
 // the wave in use (a multiple of G).
 template <int G>
 __global__ void __launch_bounds__(TPT_PLAIN_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) k_plain64(Plain64Params P) {
@@ -569,10 +569,10 @@ __global__ void __launch_bounds__(TPT_PLAIN_BLOCK) __attribute__((amdgpu_waves_p
   __shared__ int2 s_n[TPT_PLAIN_LDS * TPT_PLAIN_BLOCK];
   __shared__ double s_sh[20 * TPT_PLAIN_BLOCK];
   // domain pixel: indexes the sums and state
-  const int pix = (int)(((int64_t)blockIdx.x * P.lanes + threadIdx.x) / G);
+  const int pix = (int)(((int64_t)blockIdx.x * P.shape.lanes + threadIdx.x) / G);
   Count64 cnt{0, 0};
   uint32_t paths = 0;
-  if ((int)threadIdx.x < P.lanes && pix < P.n_pix && !P.done[pix]) {
+  if ((int)threadIdx.x < P.shape.lanes && pix < P.n_pix && !P.done[pix]) {
     PlainStack st;
     st.t_lds = s_t + threadIdx.x;
     st.n_lds = s_n + threadIdx.x;
@@ -639,7 +639,7 @@ __global__ void __launch_bounds__(TPT_PLAIN_BLOCK) __attribute__((amdgpu_waves_p
           cnt.ext++;
           vertex64(P, q, found, hit, rng, &cnt);
         }
-        if (P.mixed || !(q.env || q.light)) break;
+        if (P.shape.mixed || !(q.env || q.light)) break;
       }
       if (!(q.alive || q.env || q.light)) {  // the sample is complete
         const d3 L = q.acc;
@@ -695,29 +695,11 @@ __global__ void __launch_bounds__(TPT_PLAIN_BLOCK) __attribute__((amdgpu_waves_p
   }
 }
 
-// A pixel's samples follow each other in one random stream, so an image offers only its pixels as
-// parallel work, and the kernel (256 VGPRs, 2 waves per SIMD: 2048 waves, 131,072 lanes on the chip)
-// is bound by latency and by its divergent lanes.  With four lanes per pixel a leaf's triangles are
-// tested side by side and 16 pixels, not 64, share a wave's control flow; fewer lanes in use
-// spread few pixels over more waves.  Measured on MI355X, ms, one lane per pixel / four lanes, 64 in
-// use / four lanes, 16 in use: Cornell box 64^2 x 16 spp 5.4 / 3.6 / 2.9, 256^2 5.8 / 7.3 / 16; 82k-triangle
-// mesh 240x135 x 8 spp 18.4 / 10.9 / 6.9, 480x270 x 4 spp 11.1 / 6.9 / 9.0, 1920x1080 x 1 spp 11.0 / 18.5 / 35;
-// 64 instances 240x135 x 8 spp 21.9 / 12.9 / 13.1, 960x540 x 2 spp 11.8 / 17.4 / 34.  So four lanes up to
-// 32,768 pixels (16 in use), with deep trees up to 196,608 (64 in use).
-// mixed: one ray of any kind per turn keeps more lanes tracing but runs the shading code in every
-// turn: mesh 5% faster, Cornell box (trees of four levels at most) 18% slower.
-void plain64_shape(int depth, Plain64Params* P) {
-  const bool deep = depth >= 6, few = P->n_pix <= 32768;
-  P->mixed = deep ? 1 : 0;
-  P->quads = few || (deep && P->n_pix <= 196608) ? 1 : 0;
-  P->lanes = few ? 16 : 64;
-}
-
 hipError_t launch_plain64(const Plain64Params& P, hipStream_t s) {
   if (P.n_pix <= 0) return hipSuccess;
-  const int64_t threads = (int64_t)P.n_pix * (P.quads ? 4 : 1);
-  const dim3 grid((uint32_t)((threads + P.lanes - 1) / P.lanes)), block(TPT_PLAIN_BLOCK);
-  if (P.quads) hipLaunchKernelGGL(k_plain64<4>, grid, block, 0, s, P);
+  const int64_t threads = (int64_t)P.n_pix * (P.shape.quads ? 4 : 1);
+  const dim3 grid((uint32_t)((threads + P.shape.lanes - 1) / P.shape.lanes)), block(TPT_PLAIN_BLOCK);
+  if (P.shape.quads) hipLaunchKernelGGL(k_plain64<4>, grid, block, 0, s, P);
   else hipLaunchKernelGGL(k_plain64<1>, grid, block, 0, s, P);
   return hipGetLastError();
 }

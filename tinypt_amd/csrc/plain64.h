@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "plain64_shape.h"
 #include "tpt_kernels.h"
 
 namespace tpt {
@@ -23,10 +24,7 @@ struct Plain64Params {
   int32_t n_pix;            // pixels of the domain; domain pixel q is image pixel pix_map[q] (q if null)
   const int32_t* pix_map;
   int32_t s_begin, s_end;  // samples of this launch
-  // how the pixels are laid over the lanes (plain64_shape)
-  int32_t quads;  // a pixel has four lanes, not one
-  int32_t lanes;  // lanes of a wave in use
-  int32_t mixed;           // lanes trace shadow rays beside other lanes' extension rays
+  Plain64Shape shape;
   double threshold;
   double inv_w, inv_h;
   uint64_t seed;
@@ -41,9 +39,6 @@ struct Plain64Params {
   uint64_t* stats;  // [0] extension rays, [1] shadow rays, [2] paths
 };
 
-// Sets P's quads, lanes and mixed for P->n_pix pixels of a scene whose deepest mesh tree has
-// `depth` levels.
-void plain64_shape(int depth, Plain64Params* P);
 hipError_t launch_plain64(const Plain64Params& P, hipStream_t s);
 
 }  // namespace tpt
