@@ -498,8 +498,8 @@ int32_t refill_lanes(const HostScene& H, int32_t requested) {
   return (!H.flat && H.inst32.size() >= 64) || H.stack4 > TPT_WF_STACK ? 48 : 0;
 }
 
-// The scene as the traversal kernels for small scenes hold it; bytes 0 where it does not fit, or
-// where the caller chose how rays are handed to lanes.
+// The scene as the traversal kernels for small scenes hold it; bytes 0 where it does not fit or cannot
+// be addressed, or where the caller chose how rays are handed to lanes.
 SmallScene small_scene(const HostScene& H, int32_t requested_refill) {
   SmallScene m{};
   if (requested_refill != 0 || H.world_node0 < 0 || H.stack4 > TPT_SMALL_MAX_STACK) return m;
@@ -516,7 +516,7 @@ SmallScene small_scene(const HostScene& H, int32_t requested_refill) {
   m.n_sph = (uint32_t)sph;
   m.flat_root = H.flat ? H.inst32[(size_t)H.flat_inst].root : TPT_REF_EMPTY;
   m.stack = (uint32_t)H.stack4;
-  m.bytes = bytes;
+  if (small_scene_addressable(m)) m.bytes = bytes;
   return m;
 }
 
