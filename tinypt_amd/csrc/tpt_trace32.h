@@ -188,8 +188,8 @@ struct GlobalTree {
 // after the leaves.  The waves of a block add their gradient terms in FP32 in the order in which
 // they come to them; with the vote they come in another order, and gradients of small renders
 // moved by up to 1.5e-7 of their norm, four times what two runs differ by.  Without it they stay
-// within that.  It costs 12-bounce gradients over 20 mesh materials 2.36 -> 2.55 ms (128^2 x 16
-// spp) and the inverse step of 16 spheres 4.60 -> 4.63 (256^2 x 16 spp).
+// within that.  It costs 12-bounce gradients over 20 mesh materials 2.35 -> 2.57 ms (128^2 x 16
+// spp) and the inverse step of 16 spheres 4.60 -> 4.65 (256^2 x 16 spp).
 template <bool ANY, class Tree = GlobalTree, bool VOTE = true>
 struct TraceF32 {
   vec3<float> o, d;        // world ray
@@ -267,13 +267,11 @@ struct TraceF32 {
     bool have = true;
     for (;;) {
 #ifdef __HIP_DEVICE_COMPILE__
-      if constexpr (VOTE) {
-        const bool node = at_node();
-        if (8 * __popcll(__ballot(node)) < TPT_NODE_LANES * __popcll(__ballot(true))) break;
-        if (!node) continue;
-      } else {
-        if (!at_node()) break;
-      }
+      // one condition for both forms: with the vote in a branch of its own the compiler builds another
+      // loop around it, and the deep trees' kernels are 1.3 to 1.4 times as slow
+      const bool node = at_node();
+      if (VOTE ? 8 * __popcll(__ballot(node)) < TPT_NODE_LANES * __popcll(__ballot(true)) : !node) break;
+      if (!node) continue;
 #else
       if (!at_node()) break;
 #endif
