@@ -135,9 +135,11 @@ typedef struct tpt_stats {
   double elapsed_ms;         /* device time from first launch to last completion                */
   double trace_kernel_ms;    /* summed device time of the extension traversal kernel            */
   uint64_t trace_launches;   /* launches of the extension traversal kernel                      */
-  uint64_t trace_rays;       /* rays processed by those launches (few remaining paths are walked
-                                to their ends by a kernel of their own, whose rays count in
-                                rays_extension only)                                            */
+  uint64_t trace_rays;       /* rays processed by those launches.  Few remaining paths, and a
+                                pass of at most 2^18 paths from its start, are walked to their
+                                ends by a kernel of their own, whose rays count in
+                                rays_extension only: a render of such passes alone has 0 in
+                                these three                                                     */
   uint64_t light_samples;    /* area-light samples with a non-zero contribution (FP32 form)     */
   uint64_t light_self_occluded; /* of those, the samples whose light shadows its own surface
                                    point (integrator.rs:178-213, the reference's f64 decision)  */

@@ -94,7 +94,7 @@ struct PathSet {
   DevBuf ps_o[2], ps_d[2], ps_beta[2], ps_rng[2], ps_hit, ps_L, sh_o[2], sh_d[2], sh_c[2], sh_l, sh_lv, shl_keep, counters,
       stats, gstack;
   size_t ps_cap = 0;
-  uint64_t* seen = nullptr;  // pinned word in which a bounce's extension reports its path count (PathCount)
+  uint64_t* seen = nullptr;  // pinned word in which the first kernel after a bounce's shading reports the next bounce's paths (PathCount)
   uint64_t* seen_dev = nullptr;  // its device address
   uint32_t seen_tag = 0;         // tag of the last report asked for
   EventPool ev_trace;  // timing events of the extension launches (one call at a time)
@@ -1130,6 +1130,7 @@ int tpt_trace_closest(tpt_ctx* ctx, const tpt_scene* sc, int64_t n, const float*
   }
   return rc;
 }
+
 int tpt_trace_closest_noalloc(tpt_ctx* ctx, const tpt_scene* sc, int64_t n, const float* d_rays, float* d_hit_t,
                               int32_t* d_hit_kind, int32_t* d_hit_inst, int32_t* d_hit_prim) {
   if (!ctx || !sc || n < 0 || (n > 0 && (!d_rays || !d_hit_t || !d_hit_kind || !d_hit_inst || !d_hit_prim)))

@@ -251,10 +251,10 @@ __device__ __forceinline__ void extend_share(const WfParams& W, int cur, const T
 // waves from a global cursor stall on it, on the ray loads and, vector memory answering in order,
 // then on their next node load.  Here the nodes and triangles are in LDS, whose loads are waited
 // for apart from vector memory; a lane has its next ray in registers before it needs it (loaded
-// while the wave traces); and a wave takes rays from its own share, without atomics.  A lane's new
-// ray starts once TPT_SMALL_IDLE lanes can start one.  A ray's sequence of tests is k_extend's.
-// Cornell 512^2 x 256 spp 27.1 -> 22.3 ms (started at 8 idle lanes 23.5, 16 23.4, 32 and 48 within
-// 0.3% of 40, 56 1.5% slower); its adaptive render 28.6 -> 24.2; the inverse step's 16 spheres in
+// while the wave traces); and a wave takes rays from its own share, without atomics.  Idle lanes
+// start their rays once fewer than TPT_SMALL_LANES are tracing.  A ray's sequence of tests is
+// k_extend's.  Cornell 512^2 x 256 spp 27.1 -> 22.3 ms (below 57 tracing lanes 23.5, 49 23.4, 33 and 17
+// within 0.3% of 25, 9 1.5% slower); its adaptive render 28.6 -> 24.2; the inverse step's 16 spheres in
 // the box and the sphere scene (bound by their short launches) unchanged.
 // GEN: the first bounce's camera rays are coherent and need no loads, so a lane takes them as
 // k_extend does.
@@ -765,8 +765,8 @@ __device__ __forceinline__ void shadow_share(const WfParams& W, int queue, const
 
 // k_shadow for small scenes, see k_extend_small.
 // Cornell 512^2 x 256 spp 22.3 -> 21.5 ms; the look-ahead needs the registers of four
-// waves per SIMD (at five, with spills, 22.0; at six 23.0); started at 8 idle lanes 22.5, 32 and
-// 56 within 0.3% of 48.
+// waves per SIMD (at five, with spills, 22.0; at six 23.0); rays started below 57 tracing lanes 22.5,
+// 33 and 9 within 0.3% of 17 (TPT_SMALL_LANES_SH).
 __global__ void __launch_bounds__(TPT_WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_shadow_small(WfParams W, int queue, PathCount count) {
   extern __shared__ float4 s_small[];
@@ -916,9 +916,7 @@ __global__ void __launch_bounds__(TPT_WF_BLOCK) k_accumulate(WfParams W, AccumAr
     A.acc_w[g_pix] += (double)A.k;
     if (A.acc_sq) { A.acc_sq[3 * g_pix] += r2; A.acc_sq[3 * g_pix + 1] += g2; A.acc_sq[3 * g_pix + 2] += b2; }
   }
-  if (gtid() == 0) {
-    atomicAdd((unsigned long long*)&W.ps.stats[2], (unsigned long long)A.n_pixels * A.k);
-  }
+  if (gtid() == 0) atomicAdd((unsigned long long*)&W.ps.stats[2], (unsigned long long)A.n_pixels * A.k);
 }
 
 // Adaptive (render.rs:143-179): for each active pixel take its k new samples in sample order,

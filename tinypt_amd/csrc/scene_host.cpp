@@ -804,17 +804,9 @@ bool HostScene::build(const tpt_scene_desc* d) {
     const RefBvh& r = blas[(size_t)m];
     max_blas_depth = std::max(max_blas_depth, r.depth);
     MeshDev md{};
-    md.node_off = (int32_t)ref_nodes.size();
     md.idx_off = (int32_t)ref_indices.size();
     md.tri_off = (int32_t)b0;
-    md.n_nodes = (int32_t)r.nodes.size();
     md.n_tris = (int32_t)(b1 - b0);
-    for (const RefNode& n : r.nodes) {
-      RefNodeDev x{};
-      for (int k = 0; k < 3; k++) { x.bbox[k] = n.bbox.mn[k]; x.bbox[3 + k] = n.bbox.mx[k]; }
-      x.left = n.left; x.right = n.right; x.start = n.start; x.count = n.count;
-      ref_nodes.push_back(x);
-    }
     for (int64_t ix : r.indices) ref_indices.push_back((int32_t)ix);
     plain_meshes[(size_t)m].node_off = (int32_t)plain_nodes.size();
     if (plain_nodes.empty()) plain_nodes = std::move(plain_of[(size_t)m]);

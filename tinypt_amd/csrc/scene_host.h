@@ -83,7 +83,7 @@ struct HostScene {
   // ---- derived, FP64 (plain kernel, reference layout)
   std::vector<RefBvh> blas;
   std::vector<InstF64> inst64;       // A, t, A^-1, A^-T
-  std::vector<RefNodeDev> ref_nodes;  // all meshes' nodes, concatenated
+  std::vector<RefNodeDev> ref_nodes;  // empty: blas and plain_nodes hold the trees (the CPU tests' traversal names it)
   std::vector<int32_t> ref_indices;   // all meshes' indices (mesh-local values), concatenated
   std::vector<MeshDev> meshes;        // offsets into the concatenated arrays
   std::vector<PlainNode> plain_nodes;  // the same trees as the plain FP64 kernel walks them
@@ -124,13 +124,13 @@ struct HostScene {
   bool build(const tpt_scene_desc* d);
   void rebuild_lights();
   size_t n_tris() const { return tri_mat.size(); }
-  // Root of the flattened world-space tree when the top level holds nothing else (no spheres):
-  // rays then start there, without the top-level node and the instance entry.  Else
-  // TPT_REF_EMPTY.
   // First of the nodes and triangles that a ray meets when every ray stays in world space: the
   // flattened tree's and the top level's (spheres alone: the top level's); nodes -1 if rays enter
   // other instances.
   int64_t world_node0 = -1, world_tri0 = 0;
+  // Root of the flattened world-space tree when the top level holds nothing else (no spheres):
+  // rays then start there, without the top-level node and the instance entry.  Else
+  // TPT_REF_EMPTY.
   int32_t flat_only_root() const {
     return flat && sph_mat.empty() ? inst32[(size_t)flat_inst].root : TPT_REF_EMPTY;
   }

@@ -61,6 +61,9 @@ struct alignas(16) TriF32 {
 };
 
 struct alignas(16) InstF32 {
+  // No kernel reads these 48 B: an instance's entry takes its directions from the FP64 rows.  Taken
+  // out together with MeshDev's first two pads they cost the Cornell box 21.3 -> 21.7 ms (the
+  // shading kernel's code), so they stay.
   float w2o[12];   // rows of [A^-1 | -A^-1 t]
   float nrm[12];   // rows of A^-T (w unused)
   int32_t root;    // child ref of the mesh's BLAS root
@@ -113,10 +116,10 @@ struct InstF64 {  // transform.rs:11-20 + world.rs:39-46
 };
 
 struct MeshDev {
-  int32_t node_off;  // into the reference node array
+  int32_t pad0;
   int32_t idx_off;   // into the reference index array
   int32_t tri_off;   // into the original-order FP64 triangles
-  int32_t n_nodes;
+  int32_t pad1;
   int32_t n_tris;
   int32_t pad;
 };
