@@ -1073,7 +1073,8 @@ int tpt_render_plan(const tpt_render_config* cfg, int64_t npix, uint32_t path_bu
 }
 
 // Bound by the copies: 32 B up and 16 B down per ray, from and to pageable memory.  500k rays against a
-// 20k-triangle mesh 1.24 -> 1.01 ms, a million against 82k triangles 3.1 -> 2.3, a thousand 116 -> 110 us:
+// 20k-triangle mesh 1.24 -> 1.01 ms (the same batch again; batches in turn 1.40 -> 1.20), a million against
+// 82k triangles 3.1 -> 2.3, a thousand 116 -> 110 us:
 // buffers kept (an allocation and a release cost 10-20 us each), parts of 2^17 rays (in one part 1.07 and
 // 2.4 ms, 2^16 1.0 and 2.2 but 200k rays 0.54 instead of 0.47; one part, so no second stream, below).
 int tpt_trace_closest(tpt_ctx* ctx, const tpt_scene* sc, int64_t n, const float* rays, float* hit_t, int32_t* hit_kind,
